@@ -300,13 +300,14 @@ int xfd_device_bytes(xfd_ctx* ctx, int64_t* bytes);
 int xfd_coef_layout(xfd_ctx* ctx, int32_t* classed, int64_t* classes);
 
 /* Which CPML slabs the Yee sweeps apply in the same pass (the far grid
- * planes always stay separate launches); no reference counterpart, the
- * reference runs every slab as its own corrector (pml_corrector.h:14-52).
+ * planes, where they hold anything, are separate launches); no reference
+ * counterpart, the reference runs every slab as its own corrector
+ * (pml_corrector.h:14-52).
  *   *fused = 0: none, every slab is a separate launch;
  *   *fused = 1: the leading x/y slabs (same operations in the same order, so
  *     FP64 stays bitwise); opt-in with XFD_CPML_FUSED=1 (slower on MI355X);
- *   *fused = 2: the z slabs.  FP32: by default when a k-row spans at
- *     least 4 sweep tiles (256 cells), where it is faster; the z
+ *   *fused = 2: the z slabs.  FP32: where mode 4 does not apply and a
+ *     k-row spans at least 3 sweep tiles (more than 128 cells); the z
  *     corrections then precede the x/y slabs' where they overlap (FP32
  *     rounding only).  FP64: only when forced; the sweeps correct only the
  *     points in no x or y slab, and the frame where slabs overlap follows
@@ -320,12 +321,16 @@ int xfd_coef_layout(xfd_ctx* ctx, int32_t* classed, int64_t* classes);
  *     grid boundary plane or more than 8 slabs; XFD_CPML_FUSED=1 or
  *     XFD_CPML_ZFUSED=1 keep the two sweeps.  XFD_STEP_CHUNK (1..1024)
  *     sets the i-planes each work-item marches.
- *   *fused = 4: every slab inside the two sweeps, in boundary order per
- *     point (FP64 bitwise), each slab's parameters as kernel arguments and a
- *     point's membership from per-axis masks.  Opt-in with
- *     XFD_CPML_INSWEEP=1 (slower than modes 0 and 2 on MI355X).
- * Modes 1, 2 and 4 never with ADE materials or when a TFSF or lumped
- * correction lands inside a slab (the reference applies those first). */
+ *   *fused = 4 (the default): each half-step is one launch that applies the
+ *     update, every slab in boundary order per point (FP64 bitwise), the TFSF
+ *     and lumped corrections and the point probes.  For 3D grids, dispersive
+ *     ones included, whose slabs keep one order between every two axes, at
+ *     most two per axis, and whose corrections lie off the far planes and
+ *     outside the slabs (the reference applies those first).
+ *     XFD_CPML_INSWEEP=0 or XFD_STEP_FUSED=0 turn it off; XFD_CPML_FUSED=1 and
+ *     XFD_CPML_ZFUSED=1 select their own mode instead.
+ * Modes 1 and 2 never with ADE materials or when a TFSF or lumped correction
+ * lands inside a slab. */
 int xfd_cpml_fused(xfd_ctx* ctx, int32_t* fused);
 
 /* Zeroes a context's time-stepping state: fields, CPML auxiliaries, inductor

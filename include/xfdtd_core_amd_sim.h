@@ -45,7 +45,7 @@ int64_t xfd_sim_device_bytes(void* sim);
 /* Coefficient storage as xfd_coef_layout: 1 16-bit class ids, 2 32-bit
  * class ids, 0 dense arrays. */
 int32_t xfd_sim_coef_classed(void* sim);
-/* Which CPML slabs run inside the Yee sweeps: 0, 1 or 2 as xfd_cpml_fused. */
+/* Which CPML slabs run inside the Yee sweeps: 0 to 4 as xfd_cpml_fused. */
 int32_t xfd_sim_cpml_fused(void* sim);
 
 /* NF2FF (NFFFTFrequencyDomain) results after run() or finish(), in the

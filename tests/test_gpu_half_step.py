@@ -1,0 +1,129 @@
+"""The one-launch half-step (update, CPML slabs, TFSF and lumped corrections,
+probes) against a launch per correction, which the parity tests hold to the
+oracle bitwise: FP64 the same bits, FP32 the same up to the compiler's choice
+of contractions."""
+
+import ctypes
+
+import numpy as np
+import pytest
+
+from xfdtd_core_amd import native
+from xfdtd_core_amd import spec as S
+
+pytestmark = pytest.mark.gpu
+FIELDS = ("EX", "EY", "EZ", "HX", "HY", "HZ")
+
+
+def _box(n, pml=6, faces=("XN", "XP", "YN", "YP", "ZN", "ZP"), tfsf=True):
+    """n cells including the CPML: a lossy sphere, an inductor and a dipole,
+    a TFSF box and probes on both sides of it."""
+    dl = 1e-3
+    inner = [m - 2 * pml for m in n]
+    s = S.Simulation(dl, dl, dl, 0.9)
+    size = S.Vector(*[m * dl for m in inner])
+    s.addObject(S.Object("domain", S.Cube(S.Vector(0, 0, 0), size), S.Material.createAir()))
+    mid = [m / 2 * dl for m in inner]
+    s.addObject(S.Object("ball", S.Sphere(S.Vector(*mid), 3 * dl),
+                         S.Material("m", S.ElectroMagneticProperty(3.0, 1.0, 0.02, 0.0))))
+    cell = [m // 2 * dl for m in inner]
+    s.addObject(S.Inductor("l", S.Cube(S.Vector(cell[0] - 2 * dl, cell[1], cell[2]), S.Vector(0, 0, 2 * dl)), "Z",
+                           1e-9))
+    s.addObject(S.CurrentSource("d", S.Cube(S.Vector(*cell), S.Vector(0, 0, dl)), "ZP", 1e12,
+                                S.Waveform.gaussian(20e-12, 40e-12)))
+    if tfsf:
+        s.addWaveformSource(S.TFSF3D(pml + 2, pml + 2, pml + 2, 0.7, 0.4, 0.3, S.Waveform.gaussian(20e-12, 40e-12)))
+    for f in faces:
+        s.addBoundary(S.PML(pml, f))
+    for q, (c, comp) in enumerate(((0, "EZ"), (1, "HY"), (2, "EX"))):
+        at = [min(3 + 2 * c, m - 2) * dl for m in inner]
+        s.addMonitor(S.FieldTimeMonitor(f"p{q}", S.Cube(S.Vector(*at), S.Vector(dl, dl, dl)), "", comp))
+    return s.spec()
+
+
+def _run(monkeypatch, spec, precision, steps, on, chunk=None):
+    monkeypatch.setenv("XFD_CPML_INSWEEP", "1" if on else "0")
+    monkeypatch.setenv("XFD_CPML_ZFUSED", "0")
+    if chunk:
+        monkeypatch.setenv("XFD_ICHUNK", str(chunk))
+    sim = native.Simulation(spec, precision)
+    sim.init(steps)
+    assert sim.cpml_fused() == (4 if on else 0)
+    return sim
+
+
+def _compare(a, b, precision, label):
+    for f in FIELDS:
+        x, y = a.field(f), b.field(f)
+        assert np.abs(y).max() > 0
+        if precision == "f64":
+            np.testing.assert_array_equal(x, y, err_msg=f"{label} {f}")
+        else:
+            # each step rounds a few times at 6e-8; the two runs' roundings
+            # differ in ~50 steps, far below 1e-4 of the field's norm
+            assert np.linalg.norm(x - y) <= 1e-4 * np.linalg.norm(y), (label, f)
+
+
+# nz around the 64- and 128-lane tiles, ny off the 4-row tile, nx off the chunk
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+@pytest.mark.parametrize("n,chunk", [((23, 22, 63), None), ((24, 25, 65), 3), ((21, 23, 128), 4),
+                                     ((22, 21, 129), 1), ((30, 26, 24), 64)])
+def test_half_step_matches_separate_launches(monkeypatch, n, chunk, precision):
+    spec, steps = _box(n), 50
+    a = _run(monkeypatch, spec, precision, steps, True, chunk)
+    b = _run(monkeypatch, spec, precision, steps, False, chunk)
+    for sim in (a, b):
+        sim.advance(0, 20)
+        sim.advance(20, steps - 20)
+        sim.finish()
+    _compare(a, b, precision, f"{n} {chunk}")
+    for m in range(a.monitor_count()):
+        for x, y in zip(a.monitor_records(m), b.monitor_records(m)):
+            if precision == "f64":
+                np.testing.assert_array_equal(x, y)
+            else:
+                # a probe outside the TFSF box sees what is left of waves that
+                # cancel, so its rounding is relative to the component's peak:
+                # at most 8 roundings of 6e-8 a step in each run, 50 steps
+                peak = np.abs(b.field(("EZ", "HY", "EX")[m])).max()
+                assert np.abs(x - y).max() <= 2 * 50 * 8 * 6e-8 * peak
+
+
+# the slabs' order decides which correction a point of two slabs adds first
+@pytest.mark.parametrize("faces", [("ZN", "ZP", "YP", "YN", "XN", "XP"), ("YN", "XP", "XN"), ("ZP",), ()])
+def test_half_step_slab_orders(monkeypatch, faces):
+    spec, steps = _box((26, 24, 30), faces=faces, tfsf=len(faces) == 6), 40
+    a = _run(monkeypatch, spec, "f64", steps, True)
+    b = _run(monkeypatch, spec, "f64", steps, False)
+    for sim in (a, b):
+        sim.advance(0, steps)
+        sim.finish()
+    _compare(a, b, "f64", str(faces))
+
+
+def test_half_step_refuses_interleaved_slabs(monkeypatch):
+    """Slabs whose axes interleave in boundary order have no order per axis
+    pair: they keep a launch each."""
+    monkeypatch.setenv("XFD_CPML_INSWEEP", "1")
+    sim = native.Simulation(_box((26, 24, 30), faces=("XN", "YN", "ZN", "XP", "YP", "ZP")), "f64")
+    sim.init(2)
+    assert sim.cpml_fused() == 0
+
+
+def test_half_step_far_planes(monkeypatch):
+    """Values written on the far planes take their slab corrections."""
+    spec, steps = _box((26, 24, 30)), 30
+    runs = []
+    for on in (True, False):
+        sim = _run(monkeypatch, spec, "f64", steps, on)
+        ctx, L = sim.device_context(), native.load_library()
+        sim.advance(0, 5)
+        rng = np.random.default_rng(3)
+        for q, ext in ((0, (26, 25, 31)), (5, (26, 24, 31)), (2, (27, 25, 30))):
+            v = np.ascontiguousarray(rng.standard_normal(ext))
+            assert L.xfd_write_field(ctypes.c_void_p(ctx), q, v.ctypes.data) == 0
+        sim.advance(5, steps - 5)
+        sim.finish()
+        runs.append(sim)
+    _compare(*runs, "f64", "far planes")
+    assert np.abs(runs[0].field("EX")[:, :, -1]).max() > 0

@@ -87,9 +87,9 @@ __global__ __launch_bounds__(TK * TJ) void k_batch_sweep(const BatchCase<T>* __r
     const int by = static_cast<int>(r % C.nby);
     const int bz = static_cast<int>(r / C.nby);
     if (IsH)
-      sweepH<T, ClassCoef<T>, Fused, false, false, TK, TJ>(C.g, C.F, C.K, bx, by, bz, C.ichunk, C.ph);
+      sweepH<T, ClassCoef<T>, Fused, false, TK, TJ>(C.g, C.F, C.K, bx, by, bz, C.ichunk, C.ph);
     else
-      sweepE<T, ClassCoef<T>, Fused, false, false, TK, TJ>(C.g, C.F, C.K, bx, by, bz, C.ichunk, C.pe);
+      sweepE<T, ClassCoef<T>, Fused, false, TK, TJ>(C.g, C.F, C.K, bx, by, bz, C.ichunk, C.pe);
   }
 }
 

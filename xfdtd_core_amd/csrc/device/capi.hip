@@ -18,6 +18,7 @@
 #include "../../../include/xfdtd_core_amd.h"
 #include "adjoint_kernels.hpp"
 #include "batch_kernels.hpp"
+#include "half_step.hpp"
 #include "kernels.hpp"
 #include "step_kernels.hpp"
 
@@ -318,9 +319,15 @@ struct xfd_ctx {
   // (0: fields / psi, 1: fields_b / psi_h2).
   bool fstep = false;
   int fstep_chunk = 4;
-  // every CPML slab applied inside the two Yee sweeps (kernel-argument slab
-  // list), the far grid planes by k_cpml_faces
-  bool allslabs = false;
+  // each half-step (update, every CPML slab, records, point probes) as one
+  // launch (k_half), with its records and probes by tile
+  bool half = false;
+  int half_tk = 64, half_tj = 4, half_chunk = 4;  // tile: k-lanes x j-rows x i-planes
+  // the far planes i = nx, j = ny, k = nz hold zeros, which their slab
+  // corrections keep (they draw on each other only), so no launch visits them
+  bool far_zero = true;
+  DevBuf half_e, half_h;  // HalfSlabs of each half-step
+  DevBuf rec_off_e, seg_of_e, rec_off_h, seg_of_h, probe_off, probe_of;
   int parity = 0;
   DevBuf fields_b[6];
   bool fused = false;
@@ -650,6 +657,110 @@ bool recordsMeetSlabs(const xfd_ctx& c, const std::vector<xfd::Record>& recs, bo
 
 template <class T>
 xfd::SlabArgs<T> slabArgs(xfd_ctx::Slab& s, bool is_e);
+template <class T>
+std::vector<xfd::HalfSlabs<T>> halfSlabs(xfd_ctx& c, bool is_e);
+
+// True when the slabs of every two axes keep one order in boundary order (all
+// of one axis before all of the other), no axis has more than two slabs and
+// the two share no plane; then `swap` (HalfSlabs) describes the order.
+bool slabsByAxis(const xfd_ctx& c, int n[3], int slab[3][2], int swap[3]) {
+  for (int q = 0; q < 3; ++q) n[q] = 0;
+  for (size_t q = 0; q < c.slabs.size(); ++q) {
+    const int ax = c.slabs[q]->axis;
+    if (n[ax] == 2) return false;
+    slab[ax][n[ax]++] = static_cast<int>(q);
+  }
+  int lo[3], hi[3];
+  for (int ax = 0; ax < 3; ++ax) {
+    lo[ax] = n[ax] ? slab[ax][0] : 0;
+    hi[ax] = n[ax] ? slab[ax][n[ax] - 1] : 0;
+    if (n[ax] < 2) continue;
+    const auto &a = *c.slabs[slab[ax][0]], &b = *c.slabs[slab[ax][1]];
+    if (a.e_start < b.e_start && a.h_start < b.h_start) {
+      if (a.e_start + a.n > b.e_start || a.h_start + a.n > b.h_start) return false;
+    } else if (b.e_start + b.n <= a.e_start && b.h_start + b.n <= a.h_start) {
+      std::swap(slab[ax][0], slab[ax][1]);
+    } else {
+      return false;
+    }
+  }
+  for (int q = 0; q < 3; ++q) {
+    const int a = (q + 1) % 3, b = (q + 2) % 3;
+    swap[q] = 0;
+    if (!n[a] || !n[b]) continue;
+    if (hi[b] < lo[a])
+      swap[q] = 1;
+    else if (hi[a] > lo[b])
+      return false;
+  }
+  return true;
+}
+
+// Chooses the one-launch half-step (k_half) and lists its records and probes
+// by tile.  It takes every 3D grid but those where the order of corrections
+// would differ (a record on a point that a slab corrects, slabs that share
+// planes or interleave their axes) and those with a record on a far plane,
+// which no tile visits.  XFD_CPML_INSWEEP=0 and XFD_STEP_FUSED=0 keep a launch
+// per correction; XFD_CPML_FUSED=1 and XFD_CPML_ZFUSED=1 ask for their own.
+void halfSetup(xfd_ctx& c, const std::vector<xfd::Record>& re, const std::vector<int64_t>& se,
+               const std::vector<xfd::Record>& rh, const std::vector<int64_t>& sh,
+               const std::vector<xfd::Probe>& probes, bool records_meet_slabs) {
+  auto is = [](const char* name, char v) {
+    const char* e = std::getenv(name);
+    return e && e[0] == v;
+  };
+  const xfd::Grid& g = c.g;
+  bool far = false;
+  for (const auto* v : {&re, &rh})
+    for (const auto& r : *v) {
+      const int64_t rem = r.target % g.plane;
+      far = far || r.target / g.plane >= g.nx || rem / g.pz >= g.ny || rem % g.pz >= g.nz;
+    }
+  int n[3], slab[3][2], swap[3];
+  c.half = c.dim == 3 && !c.fstep && !records_meet_slabs && !far && slabsByAxis(c, n, slab, swap) &&
+           !is("XFD_CPML_INSWEEP", '0') && !is("XFD_STEP_FUSED", '0') && !is("XFD_CPML_FUSED", '1') &&
+           !is("XFD_CPML_ZFUSED", '1');
+  if (!c.half) return;
+  c.fused = false;
+  c.n_fused = 0;
+  c.zfused = false;
+  std::fill(c.zslab.begin(), c.zslab.end(), 0);
+  if (xfd::sweepTile128(g)) {
+    c.half_tk = 128;
+    c.half_tj = 2;
+  }
+  // up to 4 planes per work-item while about 1000 work-groups remain (100^3
+  // FP32, ms per pass: 1: 16.4, 2: 14.9, 4: 14.3, 8: 16.5; 63^3 FP64: 6.4, 6.4,
+  // 7.0, 9.9; 384^3 FP32: 482, 429, 421, 419)
+  c.half_chunk = c.ichunk;
+  if (!std::getenv("XFD_ICHUNK")) {
+    const int64_t rows = ((g.nz + 63) / 64) * ((g.ny + 3) / 4);
+    c.half_chunk = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(4, g.nx * rows / 1024)));
+  }
+  const int64_t nbx = (g.nz + c.half_tk - 1) / c.half_tk, nby = (g.ny + c.half_tj - 1) / c.half_tj;
+  const int64_t tiles = nbx * nby * ((g.nx + c.half_chunk - 1) / c.half_chunk);
+  require(tiles < (int64_t{1} << 31), "grid too large");
+  auto byTile = [&](size_t count, auto&& target, DevBuf& off, DevBuf& of) {
+    if (count == 0) return;
+    require(count < (size_t{1} << 31), "too many corrections");
+    std::vector<int32_t> o(static_cast<size_t>(tiles) + 1, 0), at(count), list(count);
+    for (size_t q = 0; q < count; ++q) {
+      const int64_t x = target(q), rem = x % g.plane;
+      const int64_t i = std::min<int64_t>(x / g.plane, g.nx - 1), j = std::min<int64_t>(rem / g.pz, g.ny - 1),
+                    k = std::min<int64_t>(rem % g.pz, g.nz - 1);
+      at[q] = static_cast<int32_t>((i / c.half_chunk * nby + j / c.half_tj) * nbx + k / c.half_tk);
+      ++o[at[q] + 1];
+    }
+    for (int64_t b = 0; b < tiles; ++b) o[b + 1] += o[b];
+    std::vector<int32_t> next(o.begin(), o.end() - 1);
+    for (size_t q = 0; q < count; ++q) list[next[at[q]]++] = static_cast<int32_t>(q);
+    uploadVector(o, off);
+    uploadVector(list, of);
+  };
+  byTile(static_cast<size_t>(c.nseg_e), [&](size_t q) { return re[se[q]].target; }, c.rec_off_e, c.seg_of_e);
+  byTile(static_cast<size_t>(c.nseg_h), [&](size_t q) { return rh[sh[q]].target; }, c.rec_off_h, c.seg_of_h);
+  byTile(probes.size(), [&](size_t q) { return probes[q].idx; }, c.probe_off, c.probe_of);
+}
 
 template <class T>
 void createTyped(xfd_ctx& c, const xfd_desc& d) {
@@ -1106,12 +1217,12 @@ void createTyped(xfd_ctx& c, const xfd_desc& d) {
     }
     c.gathers.push_back(std::move(gg));
   }
+  std::vector<xfd::Probe> probes(c.nprobe);
   if (c.nprobe) {
-    std::vector<xfd::Probe> pl(c.nprobe);
     for (auto& gg : c.gathers)
       if (gg->probe >= 0)
-        pl[gg->probe] = {padIndex(g, gg->a.o[0], gg->a.o[1], gg->a.o[2]), gg->a.field, 0};
-    uploadVector(pl, c.probe_list);
+        probes[gg->probe] = {padIndex(g, gg->a.o[0], gg->a.o[1], gg->a.o[2]), gg->a.field, 0};
+    uploadVector(probes, c.probe_list);
     c.probe_out.alloc(static_cast<size_t>(c.nprobe * c.probe_count) * sizeof(double));
   }
   if (d.n_line > 0) {  // weighted-sum recordings
@@ -1250,33 +1361,18 @@ void createTyped(xfd_ctx& c, const xfd_desc& d) {
       c.parity = 0;
     }
   }
-  {  // Every slab inside the two sweeps (boundary order per point, so FP64
-    // stays bitwise; the far planes follow in k_cpml_faces), for 3D grids
-    // without ADE, without records on points a slab corrects and with at
-    // most kMaxStepSlabs slabs.  Opt-in with XFD_CPML_INSWEEP=1: measured on
-    // the 384^3 box it is slower than the separate slab launches (FP32 1.41
-    // against 1.24 ms per step, FP64 2.27 against 2.24 ms).
-    const char* env = std::getenv("XFD_CPML_INSWEEP");
-    const char* fenv = std::getenv("XFD_CPML_FUSED");
-    const char* zenv1 = std::getenv("XFD_CPML_ZFUSED");
-    const bool other = (fenv && fenv[0] == '1') || (zenv1 && zenv1[0] == '1');
-    c.allslabs = (env && env[0] == '1') && !other && !c.fstep && c.dim == 3 && c.ade_scheme < 0 &&
-                 !records_meet_slabs && !c.slabs.empty() && c.slabs.size() <= static_cast<size_t>(xfd::kMaxStepSlabs);
-    if (c.allslabs) {
-      c.fused = false;
-      c.n_fused = 0;
-      c.zfused = false;
-      std::fill(c.zslab.begin(), c.zslab.end(), 0);
-    }
+  halfSetup(c, re, se, rh, sh, probes, records_meet_slabs);
+  if (c.half) {
+    uploadVector(halfSlabs<T>(c, true), c.half_e);
+    uploadVector(halfSlabs<T>(c, false), c.half_h);
   }
   XFD_HIP(hipStreamSynchronize(c.stream));
 }
 
-// The slabs of one half-step as the sweeps read them: in place, or for the
-// single-pass step's H side (pingpong) from the current psi set into the
-// other.
+// The slabs of one half-step as the single-pass step reads them: E in place,
+// H from the current psi set into the other.
 template <class T>
-xfd::StepSlabs<T> stepSlabs(xfd_ctx& c, bool is_e, bool pingpong = true) {
+xfd::StepSlabs<T> stepSlabs(xfd_ctx& c, bool is_e) {
   xfd::StepSlabs<T> L{};
   for (auto& sp : c.slabs) {
     const xfd::SlabArgs<T> a = slabArgs<T>(*sp, is_e);
@@ -1295,7 +1391,7 @@ xfd::StepSlabs<T> stepSlabs(xfd_ctx& c, bool is_e, bool pingpong = true) {
     S.cpsiB = a.cpsiB;
     S.ca = a.ca;
     S.cb = a.cb;
-    if (is_e || !pingpong) {
+    if (is_e) {
       S.rdA = S.wrA = a.psiA;
       S.rdB = S.wrB = a.psiB;
     } else {
@@ -1407,6 +1503,55 @@ void zCpml(xfd_ctx& c, xfd::ZCpml<T>& ze, xfd::ZCpml<T>& zh) {
 }
 
 template <class T>
+std::vector<xfd::HalfSlabs<T>> halfSlabs(xfd_ctx& c, bool is_e) {
+  std::vector<xfd::HalfSlabs<T>> v(1);
+  xfd::HalfSlabs<T>& H = v[0];
+  int slab[3][2];
+  require(slabsByAxis(c, H.n, slab, H.swap), "CPML slab order");
+  for (int ax = 0; ax < 3; ++ax)
+    for (int q = 0; q < H.n[ax]; ++q) {
+      const auto s = slabArgs<T>(*c.slabs[slab[ax][q]], is_e);
+      H.s[ax][q] = {s.start, s.start + s.n, s.ca, s.cb, s.cpsiA, s.cpsiB, s.psiA, s.psiB};
+    }
+  return v;
+}
+
+// The arguments of a context's one-launch half-step.
+template <class T>
+xfd::HalfArgs<T> halfArgs(xfd_ctx& c, bool is_e, bool probes) {
+  xfd::HalfArgs<T> a{};
+  a.slabs = (is_e ? c.half_e : c.half_h).as<xfd::HalfSlabs<T>>();
+  auto& ev = a.events;
+  if (is_e ? c.nseg_e : c.nseg_h) {
+    ev.rec_off = (is_e ? c.rec_off_e : c.rec_off_h).as<int32_t>();
+    ev.seg_of = (is_e ? c.seg_of_e : c.seg_of_h).as<int32_t>();
+    ev.rec = (is_e ? c.rec_e : c.rec_h).as<xfd::Record>();
+    ev.seg = (is_e ? c.seg_e : c.seg_h).as<int64_t>();
+    ev.nseg = is_e ? c.nseg_e : c.nseg_h;
+    ev.pool = c.pool.as<double>();
+    ev.state = c.state.as<T>();
+  }
+  if (is_e && probes && c.nprobe) {
+    ev.probe_off = c.probe_off.as<int32_t>();
+    ev.probe_of = c.probe_of.as<int32_t>();
+    ev.probe = c.probe_list.as<xfd::Probe>();
+    ev.probe_out = c.probe_out.as<double>();
+    ev.probe_count = c.probe_count;
+  }
+  a.ade = adeArgs<T>(c);
+  a.scheme = is_e ? c.ade_scheme : -1;
+  a.tk = c.half_tk;
+  a.tj = c.half_tj;
+  a.ichunk = c.half_chunk;
+  // Streamed where a step's fields and class ids exceed the 256 MB last-level
+  // cache; smaller boxes find them there in the next half-step (ms per pass
+  // plain / streamed: 100^3 FP32, 40 MB, 15.1 / 16.7; 128^3 FP64, 144 MB, 24.6 /
+  // 26.9; 203 x 181 x 225 FP64, 550 MB, 105.5 / 103.5; 384^3 FP32, 427 / 420).
+  a.stream = c.g.total * static_cast<int64_t>(6 * sizeof(T) + 12) > (int64_t{256} << 20);
+  return a;
+}
+
+template <class T>
 void stepTyped(xfd_ctx& c, int64_t t0, int64_t n, bool record = true) {
   require(t0 >= 0 && n >= 0, "bad step range");
   require(t0 + n <= c.pool_rows, "step beyond the source tables (run length given at init)");
@@ -1435,12 +1580,29 @@ void stepTyped(xfd_ctx& c, int64_t t0, int64_t n, bool record = true) {
   }
   xfd::ZCpml<T> ZE{}, ZH{};
   if (c.zfused) zCpml<T>(c, ZE, ZH);
-  xfd::StepSlabs<T> AH{}, AE{};
-  if (c.allslabs) {
-    AH = stepSlabs<T>(c, false, false);
-    AE = stepSlabs<T>(c, true, false);
+  // the one-launch half-steps; a probe may lie on a far plane, whose
+  // corrections (if any) follow the launch, so it is then sampled after them
+  const bool half_probes = record && c.far_zero;
+  xfd::HalfArgs<T> HH{}, HE{};
+  if (c.half) {
+    HH = halfArgs<T>(c, false, false);
+    HE = halfArgs<T>(c, true, half_probes);
   }
-  auto inSweep = [&](size_t q) { return c.allslabs || static_cast<int>(q) < c.n_fused; };
+  auto half = [&](bool is_e, int64_t t) {
+    const auto& a = is_e ? HE : HH;
+    c.timed(is_e ? K_UPDATE_E : K_UPDATE_H, [&] {
+      if (c.wide)
+        xfd::HalfLaunch<T>::half(st, c.g, F, M, a, is_e, t);
+      else if (c.classed)
+        xfd::HalfLaunch<T>::half(st, c.g, F, K, a, is_e, t);
+      else
+        xfd::HalfLaunch<T>::half(st, c.g, F, C, a, is_e, t);
+    });
+    if (c.far_zero) return;
+    for (const auto& sl : is_e ? se : sh)
+      c.timed(is_e ? K_CPML_E : K_CPML_H, [&] { xfd::Launch<T>::cpml_faces(st, c.g, F, sl, is_e); });
+  };
+  auto inSweep = [&](size_t q) { return static_cast<int>(q) < c.n_fused; };
   // Slabs q and q + 1 share one launch when both run separately, lie on one
   // axis and share no point (XFD_CPML_PAIR=0: one launch per slab).
   const char* pair_env = std::getenv("XFD_CPML_PAIR");
@@ -1467,6 +1629,9 @@ void stepTyped(xfd_ctx& c, int64_t t0, int64_t n, bool record = true) {
       });
       c.parity ^= 1;
       F = FB;
+    } else if (c.half) {
+      half(false, t);
+      half(true, t);
     } else {
     c.timed(K_UPDATE_H, [&] {
       if (c.dim != 3) {
@@ -1475,11 +1640,11 @@ void stepTyped(xfd_ctx& c, int64_t t0, int64_t n, bool record = true) {
         else
           xfd::Launch<T>::update_low(st, c.g, F, C, c.dim, true, c.te_zero);
       } else if (c.wide) {
-        xfd::Launch<T>::update_h(st, c.g, F, M, c.ichunk, PH, ZH, AH);
+        xfd::Launch<T>::update_h(st, c.g, F, M, c.ichunk, PH, ZH);
       } else if (c.classed) {
-        xfd::Launch<T>::update_h(st, c.g, F, K, c.ichunk, PH, ZH, AH);
+        xfd::Launch<T>::update_h(st, c.g, F, K, c.ichunk, PH, ZH);
       } else {
-        xfd::Launch<T>::update_h(st, c.g, F, C, c.ichunk, PH, ZH, AH);
+        xfd::Launch<T>::update_h(st, c.g, F, C, c.ichunk, PH, ZH);
       }
     });
     if (c.nseg_h)
@@ -1513,20 +1678,20 @@ void stepTyped(xfd_ctx& c, int64_t t0, int64_t n, bool record = true) {
         else
           xfd::Launch<T>::update_e_ade(st, c.g, F, C, A, c.ade_scheme, c.ichunk);
       } else if (c.wide) {
-        xfd::Launch<T>::update_e(st, c.g, F, M, c.ichunk, PE, ZE, AE);
+        xfd::Launch<T>::update_e(st, c.g, F, M, c.ichunk, PE, ZE);
       } else if (c.classed) {
-        xfd::Launch<T>::update_e(st, c.g, F, K, c.ichunk, PE, ZE, AE);
+        xfd::Launch<T>::update_e(st, c.g, F, K, c.ichunk, PE, ZE);
       } else {
-        xfd::Launch<T>::update_e(st, c.g, F, C, c.ichunk, PE, ZE, AE);
+        xfd::Launch<T>::update_e(st, c.g, F, C, c.ichunk, PE, ZE);
       }
     });
     }
-    if (c.nseg_e)
+    if (c.nseg_e && !c.half)
       c.timed(K_REC_E, [&] {
         xfd::Launch<T>::records(st, F, c.rec_e.as<xfd::Record>(), c.seg_e.as<int64_t>(), c.nseg_e,
                                 c.pool.as<double>(), c.state.as<T>(), t);
       });
-    for (size_t q = 0; q < se.size() && !c.fstep; ++q)
+    for (size_t q = 0; q < se.size() && !c.fstep && !c.half; ++q)
       c.timed(K_CPML_E, [&] {
         if (pairs(se, q)) {
           xfd::Launch<T>::cpml2(st, c.g, F, se[q], se[q + 1], true);
@@ -1542,7 +1707,7 @@ void stepTyped(xfd_ctx& c, int64_t t0, int64_t n, bool record = true) {
       XFD_HIP(hipGetLastError());
       continue;
     }
-    if (c.nprobe && t < c.probe_count)
+    if (c.nprobe && t < c.probe_count && !(c.half && half_probes))
       c.timed(K_GATHER, [&] {
         xfd::Launch<T>::probes(st, F, c.probe_list.as<xfd::Probe>(), c.nprobe, c.probe_out.as<double>(),
                                c.probe_count, t);
@@ -1596,6 +1761,7 @@ void stepTyped(xfd_ctx& c, int64_t t0, int64_t n, bool record = true) {
 // Zeroes every piece of time-stepping state of a case: fields, CPML psi,
 // inductor currents, ADE state, NF2FF accumulators and recordings.
 void resetState(xfd_ctx& c) {
+  c.far_zero = true;
   auto zero = [&](DevBuf& b) {
     if (b.p && b.bytes) XFD_HIP(hipMemsetAsync(b.p, 0, b.bytes, c.stream));
   };
@@ -2355,6 +2521,16 @@ int xfd_write_field(xfd_ctx* c, int32_t field, const double* src) {
     if (field == 0 || field == 1 || field == 5) c->te_zero = false;  // no longer known to stay zero
     int ext[3];
     extentOf(field, c->g.nx, c->g.ny, c->g.nz, ext);
+    if (c->half && c->far_zero) {  // a far plane that no longer holds zeros takes its slab corrections
+      const int n[3] = {c->g.nx, c->g.ny, c->g.nz};
+      bool zero = true;
+      for (int i = 0; i < ext[0] && zero; ++i)
+        for (int j = 0; j < ext[1] && zero; ++j) {
+          const double* row = src + (static_cast<int64_t>(i) * ext[1] + j) * ext[2];
+          for (int k = i == n[0] || j == n[1] ? 0 : n[2]; k < ext[2]; ++k) zero = zero && row[k] == 0.0;
+        }
+      c->far_zero = zero;
+    }
     DevBuf tmp;
     tmp.alloc(static_cast<size_t>(ext[0]) * ext[1] * ext[2] * sizeof(double));
     DevBuf& cur = curFields(*c)[field];
@@ -2592,7 +2768,7 @@ int xfd_nf2ff_far_field_noalloc(xfd_ctx* c, int32_t n, int32_t f, int32_t na, co
 int xfd_cpml_fused(xfd_ctx* c, int32_t* fused) {
   return guard([&] {
     require(c && fused, "bad argument");
-    *fused = c->fstep ? 3 : (c->allslabs ? 4 : (c->fused ? 1 : (c->zfused ? 2 : 0)));
+    *fused = c->fstep ? 3 : (c->half ? 4 : (c->fused ? 1 : (c->zfused ? 2 : 0)));
   });
 }
 
@@ -2620,7 +2796,7 @@ int xfd_batch_create(int32_t n, const xfd_desc* descs, xfd_batch** out) {
       if (xfd_create(&descs[i], &c) != XFD_OK) throw XfdError(XFD_EINVAL, std::string("case ") + std::to_string(i) + ": " + g_err);
       b->cases.emplace_back(c);
       leaveStep(*c);  // the batched launches step set 0 with their own tables
-      c->allslabs = false;
+      c->half = false;
       // batched cases keep their z slabs as separate launches: with most
       // wavefronts of these small boxes carrying slab lanes, the sweeps were
       // measured slower with them inside

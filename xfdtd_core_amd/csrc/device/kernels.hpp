@@ -15,6 +15,8 @@
 // reference's CPU path; the FP32 unit lets the compiler fuse.
 #pragma once
 
+#include <cstdlib>
+
 #include "layout.hpp"
 #include "slab_inline.hpp"
 
@@ -193,11 +195,10 @@ __device__ __forceinline__ void zStore(const ZCpml<T>& Z, const ZLane<T>& L, con
 // One work-group tile: k-block bx, j-block by, i-chunk bz.  Fused: the CPML
 // H corrections of the visited points in the same pass (the H dual
 // differences along x, y, z are dual[idx + s_c] - dual[idx]).
-template <class T, class Coef, bool Fused = false, bool ZF = false, bool All = false, int TK = kLanesK,
-          int TJ = kRowsJ>
+template <class T, class Coef, bool Fused = false, bool ZF = false, int TK = kLanesK, int TJ = kRowsJ>
 __device__ __forceinline__ void sweepH(const Grid& g, const FieldPtrs<T>& F, const Coef& C, int bx, int by, int bz,
                                        int ichunk, const CpmlList<T>& P = CpmlList<T>{},
-                                       const ZCpml<T>& Z = ZCpml<T>{}, const StepSlabs<T>& S = StepSlabs<T>{}) {
+                                       const ZCpml<T>& Z = ZCpml<T>{}) {
   const int k = bx * TK + threadIdx.x;
   const int j = by * TJ + threadIdx.y;
   const int i0 = bz * ichunk;
@@ -216,9 +217,6 @@ __device__ __forceinline__ void sweepH(const Grid& g, const FieldPtrs<T>& F, con
   const uint32_t mask = Fused ? cpmlChunkMask(P, i0, i1, j, k) : 0u;
   ZLane<T> zl;
   if (ZF) zl = zLane(Z, i0, j, k);
-  // All: every slab of S (its j and k masks, the k mask's wavefront union)
-  const uint32_t sj = All ? axisMask(S, 1, j) : 0u, sk = All ? axisMask(S, 2, k) : 0u;
-  const uint32_t sku = All ? waveUnion(sk) : 0u;
   for (int i = i0; i < i1; ++i, idx += pl) {
     ZVals<T> zv;
     if (ZF) zv = zLoad<T, false>(Z, zl, i, nullptr, nullptr, idx);
@@ -239,12 +237,6 @@ __device__ __forceinline__ void sweepH(const Grid& g, const FieldPtrs<T>& F, con
       zStore(Z, zl, zv, vx, vy, ey_k - ey_i, ex_k - ex0);
       zl.t += zl.step;
     }
-    if (All) {
-      const uint32_t si = axisMask(S, 0, i) & sj;
-      if (si & sku)
-        stepSlabs<T, true>(S, si & sku, si & sk, i, j, k, vx, vy, vz, ez_n - ez_i, ex_j - ex0, ey_k - ey_i,
-                           ey_n - ey_i, ez_j - ez_i, ex_k - ex0);
-    }
     stOwn(hx + idx, vx);
     stOwn(hy + idx, vy);
     stOwn(hz + idx, vz);
@@ -253,12 +245,12 @@ __device__ __forceinline__ void sweepH(const Grid& g, const FieldPtrs<T>& F, con
   }
 }
 
-template <class T, class Coef, bool Fused, bool ZF, bool All, int TK = kLanesK, int TJ = kRowsJ>
+template <class T, class Coef, bool Fused, bool ZF, int TK = kLanesK, int TJ = kRowsJ>
 __global__ __launch_bounds__(TK * TJ) void k_update_h(Grid g, FieldPtrs<T> F, Coef C, SweepMap M, int ichunk,
-                                             CpmlList<T> P, ZCpml<T> Z, StepSlabs<T> S) {
+                                             CpmlList<T> P, ZCpml<T> Z) {
   int bx, by, bz;
   M.coords(bx, by, bz);
-  sweepH<T, Coef, Fused, ZF, All, TK, TJ>(g, F, C, bx, by, bz, ichunk, P, Z, S);
+  sweepH<T, Coef, Fused, ZF, TK, TJ>(g, F, C, bx, by, bz, ichunk, P, Z);
 }
 
 // BasicUpdator3D::updateE (src/updator/basic_updator_3d.cpp:38-69):
@@ -267,11 +259,10 @@ __global__ __launch_bounds__(TK * TJ) void k_update_h(Grid g, FieldPtrs<T> F, Co
 // visited points (i < nx, j < ny, k < nz) in the same pass, including the
 // face points a Yee range leaves out; the dual differences along x, y, z are
 // dual[idx] - dual[idx - s_c].
-template <class T, class Coef, bool Fused = false, bool ZF = false, bool All = false, int TK = kLanesK,
-          int TJ = kRowsJ>
+template <class T, class Coef, bool Fused = false, bool ZF = false, int TK = kLanesK, int TJ = kRowsJ>
 __device__ __forceinline__ void sweepE(const Grid& g, const FieldPtrs<T>& F, const Coef& C, int bx, int by, int bz,
                                        int ichunk, const CpmlList<T>& P = CpmlList<T>{},
-                                       const ZCpml<T>& Z = ZCpml<T>{}, const StepSlabs<T>& S = StepSlabs<T>{}) {
+                                       const ZCpml<T>& Z = ZCpml<T>{}) {
   const int k = bx * TK + threadIdx.x;
   const int j = by * TJ + threadIdx.y;
   const int i0 = bz * ichunk;
@@ -292,15 +283,12 @@ __device__ __forceinline__ void sweepE(const Grid& g, const FieldPtrs<T>& F, con
   const uint32_t mask = Fused ? cpmlChunkMask(P, i0, i1, j, k) : 0u;
   ZLane<T> zl;
   if (ZF) zl = zLane(Z, i0, j, k);
-  const uint32_t sj = All ? axisMask(S, 1, j) : 0u, sk = All ? axisMask(S, 2, k) : 0u;
-  const uint32_t sku = All ? waveUnion(sk) : 0u;
   for (int i = i0; i < i1; ++i, idx += pl) {
     ZVals<T> zv;
     if (ZF) zv = zLoad<T, true>(Z, zl, i, hy, hx, idx);  // Ex <- Hy, Ey <- Hx (k >= 1 in a z slab)
     const T hx0 = hx[idx], hy0 = hy[idx], hz0 = hz[idx];
     T s, a, b;
-    const uint32_t si = All ? axisMask(S, 0, i) & sj : 0u;
-    if (All ? !(si & sku) : (!Fused || !mask)) {
+    if (!Fused || !mask) {
       // every lane stores its three values (unchanged on the faces the Yee
       // ranges leave out), so each wavefront writes whole lines: skipping the
       // j = 0 / k = 0 lanes left partial lines and cost 6 % of the FP32 sweep.
@@ -349,10 +337,7 @@ __device__ __forceinline__ void sweepE(const Grid& g, const FieldPtrs<T>& F, con
         vz = s * vz + a * dyHx + b * dxHy;
       }
       // A: Ey(x) <- Hz, Ez(y) <- Hx, Ex(z) <- Hy;  B: Ez(x) <- Hy, Ex(y) <- Hz, Ey(z) <- Hx
-      if (All)
-        stepSlabs<T, true>(S, si & sku, si & sk, i, j, k, vx, vy, vz, dxHz, dyHx, dzHy, dxHy, dyHz, dzHx);
-      else
-        cpmlFused(P, mask, i, j, k, vx, vy, vz, dxHz, dyHx, dzHy, dxHy, dyHz, dzHx);
+      cpmlFused(P, mask, i, j, k, vx, vy, vz, dxHz, dyHx, dzHy, dxHy, dyHz, dzHx);
       ex[idx] = vx;
       ey[idx] = vy;
       ez[idx] = vz;
@@ -362,12 +347,12 @@ __device__ __forceinline__ void sweepE(const Grid& g, const FieldPtrs<T>& F, con
   }
 }
 
-template <class T, class Coef, bool Fused, bool ZF, bool All, int TK = kLanesK, int TJ = kRowsJ>
+template <class T, class Coef, bool Fused, bool ZF, int TK = kLanesK, int TJ = kRowsJ>
 __global__ __launch_bounds__(TK * TJ) void k_update_e(Grid g, FieldPtrs<T> F, Coef C, SweepMap M, int ichunk,
-                                             CpmlList<T> P, ZCpml<T> Z, StepSlabs<T> S) {
+                                             CpmlList<T> P, ZCpml<T> Z) {
   int bx, by, bz;
   M.coords(bx, by, bz);
-  sweepE<T, Coef, Fused, ZF, All, TK, TJ>(g, F, C, bx, by, bz, ichunk, P, Z, S);
+  sweepE<T, Coef, Fused, ZF, TK, TJ>(g, F, C, bx, by, bz, ichunk, P, Z);
 }
 
 // 2D (TE) grid, nz = 1, in a layout of pitch pz = 2 along k (k = 1 holds
@@ -1235,32 +1220,35 @@ __global__ __launch_bounds__(256) void k_td_bins_wave(TdNf2ffArgs a, int64_t t) 
   tdBinWave(a, g / 64, static_cast<int>(g % 64), t);
 }
 
+// The plain and z-in-sweep Yee sweeps take 128 k-lanes x 2 j-rows where nz
+// is a multiple of 128 (no idle lanes; half the k-halo loads per point of a
+// 64-lane row): measured on the 384^3 box, ms per step FP32 / FP64, 64 x 4
+// 1.115 / 2.216, 128 x 2 1.088 / 2.183.  Elsewhere 64 x 4, whose rows waste
+// fewer lanes on ragged nz.  XFD_SWEEP_TILE=64 / 128 forces one of them.
+inline bool sweepTile128(const Grid& g) {
+  const char* e = std::getenv("XFD_SWEEP_TILE");
+  if (e && e[0]) return std::atoi(e) == 128;
+  return g.nz % 128 == 0;
+}
+
 // Host-side launchers, instantiated once per precision.
 template <class T>
 struct Launch {
   // P.n > 0: the sweep applies the slabs of P in the same pass; Z.n > 0:
   // the sweep applies the z slabs of Z (then cpml_faces completes either on
   // the far grid planes)
-  // S.n > 0: the sweep applies every slab of S (in boundary order; P and Z
-  // unused)
   static void update_h(hipStream_t s, const Grid& g, const FieldPtrs<T>& F, const CoefPtrs<T>& C, int ichunk,
-                       const CpmlList<T>& P = CpmlList<T>{}, const ZCpml<T>& Z = ZCpml<T>{},
-                       const StepSlabs<T>& S = StepSlabs<T>{});
+                       const CpmlList<T>& P = CpmlList<T>{}, const ZCpml<T>& Z = ZCpml<T>{});
   static void update_e(hipStream_t s, const Grid& g, const FieldPtrs<T>& F, const CoefPtrs<T>& C, int ichunk,
-                       const CpmlList<T>& P = CpmlList<T>{}, const ZCpml<T>& Z = ZCpml<T>{},
-                       const StepSlabs<T>& S = StepSlabs<T>{});
+                       const CpmlList<T>& P = CpmlList<T>{}, const ZCpml<T>& Z = ZCpml<T>{});
   static void update_h(hipStream_t s, const Grid& g, const FieldPtrs<T>& F, const ClassCoef<T>& C, int ichunk,
-                       const CpmlList<T>& P = CpmlList<T>{}, const ZCpml<T>& Z = ZCpml<T>{},
-                       const StepSlabs<T>& S = StepSlabs<T>{});
+                       const CpmlList<T>& P = CpmlList<T>{}, const ZCpml<T>& Z = ZCpml<T>{});
   static void update_e(hipStream_t s, const Grid& g, const FieldPtrs<T>& F, const ClassCoef<T>& C, int ichunk,
-                       const CpmlList<T>& P = CpmlList<T>{}, const ZCpml<T>& Z = ZCpml<T>{},
-                       const StepSlabs<T>& S = StepSlabs<T>{});
+                       const CpmlList<T>& P = CpmlList<T>{}, const ZCpml<T>& Z = ZCpml<T>{});
   static void update_h(hipStream_t s, const Grid& g, const FieldPtrs<T>& F, const WideCoef<T>& C, int ichunk,
-                       const CpmlList<T>& P = CpmlList<T>{}, const ZCpml<T>& Z = ZCpml<T>{},
-                       const StepSlabs<T>& S = StepSlabs<T>{});
+                       const CpmlList<T>& P = CpmlList<T>{}, const ZCpml<T>& Z = ZCpml<T>{});
   static void update_e(hipStream_t s, const Grid& g, const FieldPtrs<T>& F, const WideCoef<T>& C, int ichunk,
-                       const CpmlList<T>& P = CpmlList<T>{}, const ZCpml<T>& Z = ZCpml<T>{},
-                       const StepSlabs<T>& S = StepSlabs<T>{});
+                       const CpmlList<T>& P = CpmlList<T>{}, const ZCpml<T>& Z = ZCpml<T>{});
   // the Yee half-steps of a 2D (TE, dim 2) or 1D (TEM, dim 1) grid; the 1D
   // H half-step is the 3D sweep (update_h)
   // te_zero (2D): Ex, Ey and Hz are known to stay zero, so the H half-step

@@ -6,3 +6,4 @@ template struct xfd::Launch<double>;
 template struct xfd::BatchLaunch<double>;
 template struct xfd::AdjLaunch<double>;
 template struct xfd::StepLaunch<double>;
+template struct xfd::HalfLaunch<double>;

@@ -8,6 +8,7 @@
 
 #include "adjoint_kernels.hpp"
 #include "batch_kernels.hpp"
+#include "half_step.hpp"
 #include "kernels.hpp"
 #include "step_kernels.hpp"
 
@@ -27,76 +28,63 @@ inline SweepMap sweepMap(const Grid& g, int ichunk, int tk = kLanesK, int tj = k
                   static_cast<int>(blocks_for(g.nx, ichunk)), xcd};
 }
 
-// The plain and z-in-sweep Yee sweeps take 128 k-lanes x 2 j-rows where nz
-// is a multiple of 128 (no idle lanes; half the k-halo loads per point of a
-// 64-lane row): measured on the 384^3 box, ms per step FP32 / FP64, 64 x 4
-// 1.115 / 2.216, 128 x 2 1.088 / 2.183.  Elsewhere 64 x 4, whose rows waste
-// fewer lanes on ragged nz.  XFD_SWEEP_TILE=64 / 128 forces one of them.
-inline bool sweepTile128(const Grid& g) {
-  const char* e = std::getenv("XFD_SWEEP_TILE");
-  if (e && e[0]) return std::atoi(e) == 128;
-  return g.nz % 128 == 0;
-}
-
-template <class T, class Coef, bool Fused, bool ZF, bool All, int TK, int TJ>
+template <class T, class Coef, bool Fused, bool ZF, int TK, int TJ>
 void launchSweep(bool is_h, hipStream_t s, const Grid& g, const FieldPtrs<T>& F, const Coef& C, int ichunk,
-                 const CpmlList<T>& P, const ZCpml<T>& Z, const StepSlabs<T>& S) {
+                 const CpmlList<T>& P, const ZCpml<T>& Z) {
   const SweepMap m = sweepMap(g, ichunk, TK, TJ);
   const dim3 grid(static_cast<unsigned>(m.nbx * m.nby * m.nbz)), block(TK, TJ);
   if (is_h)
-    hipLaunchKernelGGL((k_update_h<T, Coef, Fused, ZF, All, TK, TJ>), grid, block, 0, s, g, F, C, m, ichunk, P, Z, S);
+    hipLaunchKernelGGL((k_update_h<T, Coef, Fused, ZF, TK, TJ>), grid, block, 0, s, g, F, C, m, ichunk, P, Z);
   else
-    hipLaunchKernelGGL((k_update_e<T, Coef, Fused, ZF, All, TK, TJ>), grid, block, 0, s, g, F, C, m, ichunk, P, Z, S);
+    hipLaunchKernelGGL((k_update_e<T, Coef, Fused, ZF, TK, TJ>), grid, block, 0, s, g, F, C, m, ichunk, P, Z);
 }
 
 template <class T, class Coef>
 void launchUpdate(bool is_h, hipStream_t s, const Grid& g, const FieldPtrs<T>& F, const Coef& C, int ichunk,
-                  const CpmlList<T>& P, const ZCpml<T>& Z, const StepSlabs<T>& S = StepSlabs<T>{}) {
-  const bool all = S.n > 0, fused = !all && P.n > 0, zf = !all && !fused && Z.n > 0;
-  const bool t128 = !all && !fused && sweepTile128(g);
-  if (all)
-    launchSweep<T, Coef, false, false, true, kLanesK, kRowsJ>(is_h, s, g, F, C, ichunk, P, Z, S);
-  else if (fused)
-    launchSweep<T, Coef, true, false, false, kLanesK, kRowsJ>(is_h, s, g, F, C, ichunk, P, Z, S);
+                  const CpmlList<T>& P, const ZCpml<T>& Z) {
+  const bool fused = P.n > 0, zf = !fused && Z.n > 0;
+  const bool t128 = !fused && sweepTile128(g);
+  if (fused)
+    launchSweep<T, Coef, true, false, kLanesK, kRowsJ>(is_h, s, g, F, C, ichunk, P, Z);
   else if (zf && t128)
-    launchSweep<T, Coef, false, true, false, 128, 2>(is_h, s, g, F, C, ichunk, P, Z, S);
+    launchSweep<T, Coef, false, true, 128, 2>(is_h, s, g, F, C, ichunk, P, Z);
   else if (zf)
-    launchSweep<T, Coef, false, true, false, kLanesK, kRowsJ>(is_h, s, g, F, C, ichunk, P, Z, S);
+    launchSweep<T, Coef, false, true, kLanesK, kRowsJ>(is_h, s, g, F, C, ichunk, P, Z);
   else if (t128)
-    launchSweep<T, Coef, false, false, false, 128, 2>(is_h, s, g, F, C, ichunk, P, Z, S);
+    launchSweep<T, Coef, false, false, 128, 2>(is_h, s, g, F, C, ichunk, P, Z);
   else
-    launchSweep<T, Coef, false, false, false, kLanesK, kRowsJ>(is_h, s, g, F, C, ichunk, P, Z, S);
+    launchSweep<T, Coef, false, false, kLanesK, kRowsJ>(is_h, s, g, F, C, ichunk, P, Z);
 }
 
 template <class T>
 void Launch<T>::update_h(hipStream_t s, const Grid& g, const FieldPtrs<T>& F, const CoefPtrs<T>& C, int ichunk,
-                         const CpmlList<T>& P, const ZCpml<T>& Z, const StepSlabs<T>& S) {
-  launchUpdate<T>(true, s, g, F, C, ichunk, P, Z, S);
+                         const CpmlList<T>& P, const ZCpml<T>& Z) {
+  launchUpdate<T>(true, s, g, F, C, ichunk, P, Z);
 }
 template <class T>
 void Launch<T>::update_e(hipStream_t s, const Grid& g, const FieldPtrs<T>& F, const CoefPtrs<T>& C, int ichunk,
-                         const CpmlList<T>& P, const ZCpml<T>& Z, const StepSlabs<T>& S) {
-  launchUpdate<T>(false, s, g, F, C, ichunk, P, Z, S);
+                         const CpmlList<T>& P, const ZCpml<T>& Z) {
+  launchUpdate<T>(false, s, g, F, C, ichunk, P, Z);
 }
 template <class T>
 void Launch<T>::update_h(hipStream_t s, const Grid& g, const FieldPtrs<T>& F, const ClassCoef<T>& C, int ichunk,
-                         const CpmlList<T>& P, const ZCpml<T>& Z, const StepSlabs<T>& S) {
-  launchUpdate<T>(true, s, g, F, C, ichunk, P, Z, S);
+                         const CpmlList<T>& P, const ZCpml<T>& Z) {
+  launchUpdate<T>(true, s, g, F, C, ichunk, P, Z);
 }
 template <class T>
 void Launch<T>::update_e(hipStream_t s, const Grid& g, const FieldPtrs<T>& F, const ClassCoef<T>& C, int ichunk,
-                         const CpmlList<T>& P, const ZCpml<T>& Z, const StepSlabs<T>& S) {
-  launchUpdate<T>(false, s, g, F, C, ichunk, P, Z, S);
+                         const CpmlList<T>& P, const ZCpml<T>& Z) {
+  launchUpdate<T>(false, s, g, F, C, ichunk, P, Z);
 }
 template <class T>
 void Launch<T>::update_h(hipStream_t s, const Grid& g, const FieldPtrs<T>& F, const WideCoef<T>& C, int ichunk,
-                         const CpmlList<T>& P, const ZCpml<T>& Z, const StepSlabs<T>& S) {
-  launchUpdate<T>(true, s, g, F, C, ichunk, P, Z, S);
+                         const CpmlList<T>& P, const ZCpml<T>& Z) {
+  launchUpdate<T>(true, s, g, F, C, ichunk, P, Z);
 }
 template <class T>
 void Launch<T>::update_e(hipStream_t s, const Grid& g, const FieldPtrs<T>& F, const WideCoef<T>& C, int ichunk,
-                         const CpmlList<T>& P, const ZCpml<T>& Z, const StepSlabs<T>& S) {
-  launchUpdate<T>(false, s, g, F, C, ichunk, P, Z, S);
+                         const CpmlList<T>& P, const ZCpml<T>& Z) {
+  launchUpdate<T>(false, s, g, F, C, ichunk, P, Z);
 }
 template <class T, class Coef>
 void launchLow(hipStream_t s, const Grid& g, const FieldPtrs<T>& F, const Coef& C, int dim, bool is_h,
@@ -541,6 +529,53 @@ template <class T>
 void StepLaunch<T>::step(hipStream_t s, const Grid& g, const FieldPtrs<T>& A, const FieldPtrs<T>& B,
                          const ClassCoef<T>& C, const StepSlabs<T>& SH, const StepSlabs<T>& SE, int ichunk) {
   launchStep<T>(s, g, A, B, C, SH, SE, ichunk);
+}
+
+template <class T, class Coef, bool NT, int TK, int TJ>
+void launchHalf(hipStream_t s, const Grid& g, const FieldPtrs<T>& F, const Coef& C, const HalfArgs<T>& a, bool is_e,
+                int64_t t) {
+  const SweepMap m = sweepMap(g, a.ichunk, TK, TJ);
+  const dim3 grid(static_cast<unsigned>(m.nbx * m.nby * m.nbz)), block(TK, TJ);
+  if (!is_e)
+    hipLaunchKernelGGL((k_half<T, Coef, false, -1, NT, TK, TJ>), grid, block, 0, s, g, F, C, a.ade, a.slabs, a.events, m,
+                       a.ichunk, t);
+  else if (a.scheme < 0)
+    hipLaunchKernelGGL((k_half<T, Coef, true, -1, NT, TK, TJ>), grid, block, 0, s, g, F, C, a.ade, a.slabs, a.events, m,
+                       a.ichunk, t);
+  else if (a.scheme == kAdeDrude)
+    hipLaunchKernelGGL((k_half<T, Coef, true, kAdeDrude, NT, TK, TJ>), grid, block, 0, s, g, F, C, a.ade, a.slabs,
+                       a.events, m, a.ichunk, t);
+  else if (a.scheme == kAdeDebye)
+    hipLaunchKernelGGL((k_half<T, Coef, true, kAdeDebye, NT, TK, TJ>), grid, block, 0, s, g, F, C, a.ade, a.slabs,
+                       a.events, m, a.ichunk, t);
+  else
+    hipLaunchKernelGGL((k_half<T, Coef, true, kAdeMLorentz, NT, TK, TJ>), grid, block, 0, s, g, F, C, a.ade, a.slabs,
+                       a.events, m, a.ichunk, t);
+}
+template <class T, class Coef>
+void launchHalfTile(hipStream_t s, const Grid& g, const FieldPtrs<T>& F, const Coef& C, const HalfArgs<T>& a,
+                    bool is_e, int64_t t) {
+  if (a.tk == 128)
+    a.stream ? launchHalf<T, Coef, true, 128, 2>(s, g, F, C, a, is_e, t)
+             : launchHalf<T, Coef, false, 128, 2>(s, g, F, C, a, is_e, t);
+  else
+    a.stream ? launchHalf<T, Coef, true, kLanesK, kRowsJ>(s, g, F, C, a, is_e, t)
+             : launchHalf<T, Coef, false, kLanesK, kRowsJ>(s, g, F, C, a, is_e, t);
+}
+template <class T>
+void HalfLaunch<T>::half(hipStream_t s, const Grid& g, const FieldPtrs<T>& F, const CoefPtrs<T>& C,
+                         const HalfArgs<T>& a, bool is_e, int64_t t) {
+  launchHalfTile<T>(s, g, F, C, a, is_e, t);
+}
+template <class T>
+void HalfLaunch<T>::half(hipStream_t s, const Grid& g, const FieldPtrs<T>& F, const ClassCoef<T>& C,
+                         const HalfArgs<T>& a, bool is_e, int64_t t) {
+  launchHalfTile<T>(s, g, F, C, a, is_e, t);
+}
+template <class T>
+void HalfLaunch<T>::half(hipStream_t s, const Grid& g, const FieldPtrs<T>& F, const WideCoef<T>& C,
+                         const HalfArgs<T>& a, bool is_e, int64_t t) {
+  launchHalfTile<T>(s, g, F, C, a, is_e, t);
 }
 
 }  // namespace xfd

@@ -55,28 +55,23 @@ struct FieldPtrs {
 };
 
 // Streamed per-cell data (own fields, class ids, CPML psi: read and written
-// once per pass) carries the non-temporal hint, so it does not displace the
-// neighbour rows other work-groups still read from L2 (measured on the 384^3
-// box: FP32 +5 %, FP64 +9 %; batched sweep +13 %).  XFD_STREAMING_OWN=0 at
-// build time turns it off.
-#ifndef XFD_STREAMING_OWN
-#define XFD_STREAMING_OWN 1
-#endif
-template <class T>
+// once per pass) carries the non-temporal hint where a step moves more than
+// the caches hold, so it does not displace the neighbour rows other
+// work-groups still read from L2 (measured on the 384^3 box: FP32 +5 %, FP64
+// +9 %; batched sweep +13 %).  NT = false: plain accesses.
+template <bool NT = true, class T>
 __device__ __forceinline__ T ldOwn(const T* p) {
-#if XFD_STREAMING_OWN
-  return __builtin_nontemporal_load(p);
-#else
-  return *p;
-#endif
+  if constexpr (NT)
+    return __builtin_nontemporal_load(p);
+  else
+    return *p;
 }
-template <class T>
+template <bool NT = true, class T>
 __device__ __forceinline__ void stOwn(T* p, T v) {
-#if XFD_STREAMING_OWN
-  __builtin_nontemporal_store(v, p);
-#else
-  *p = v;
-#endif
+  if constexpr (NT)
+    __builtin_nontemporal_store(v, p);
+  else
+    *p = v;
 }
 
 // Coefficient access for component q (0..5 = Ex Ey Ez Hx Hy Hz): the
@@ -102,8 +97,9 @@ struct CoefPtrs {
   struct Raw {
     T s, a, b;
   };
+  template <bool NT = true>
   __device__ __forceinline__ Raw raw(int q, int64_t idx) const {
-    return Raw{ldOwn(c[3 * q] + idx), ldOwn(c[3 * q + 1] + idx), ldOwn(c[3 * q + 2] + idx)};
+    return Raw{ldOwn<NT>(c[3 * q] + idx), ldOwn<NT>(c[3 * q + 1] + idx), ldOwn<NT>(c[3 * q + 2] + idx)};
   }
   __device__ __forceinline__ void resolve(int, const Raw& r, T& s, T& a, T& b) const {
     s = r.s;
@@ -134,7 +130,10 @@ struct ClassCoef {
   struct Raw {
     int id;
   };
-  __device__ __forceinline__ Raw raw(int q, int64_t idx) const { return Raw{static_cast<int>(ldOwn(id[q] + idx))}; }
+  template <bool NT = true>
+  __device__ __forceinline__ Raw raw(int q, int64_t idx) const {
+    return Raw{static_cast<int>(ldOwn<NT>(id[q] + idx))};
+  }
   __device__ __forceinline__ void resolve(int q, const Raw& r, T& s, T& a, T& b) const {
     const T* e = tab[q] + 3 * r.id;
     s = e[0];

@@ -390,9 +390,10 @@ class Simulation:
 
     def cpml_fused(self) -> int:
         """Which CPML slabs the Yee sweeps apply in the same pass: 0 none,
-        1 the leading x/y slabs (XFD_CPML_FUSED=1), 2 the z slabs (FP32
-        when nz > 192; either precision with XFD_CPML_ZFUSED=1; =0 turns it
-        off)."""
+        1 the leading x/y slabs (XFD_CPML_FUSED=1), 2 the z slabs
+        (XFD_CPML_ZFUSED=1, or FP32 with nz > 128 where 4 does not apply), 3
+        all in the single-pass step (XFD_STEP_FUSED=1), 4 all, with the other
+        corrections, in one launch per half-step (the default)."""
         return int(self._L.xfd_sim_cpml_fused(self._h))
 
     def coef_classed(self) -> bool:
