@@ -1,0 +1,66 @@
+"""1D grids stepped many times per launch against a launch per correction,
+which the low-dimension tests hold to the oracle: FP64 the same bits, FP32 up to
+the compiler's choice of contractions."""
+
+import numpy as np
+import pytest
+
+from xfdtd_core_amd import native
+from xfdtd_core_amd import spec as S
+
+pytestmark = pytest.mark.gpu
+INF = float("inf")
+
+
+def _line(nz, tfsf=5, pml=8, faces=("ZN", "ZP")):
+    dl = 1e-3
+    s = S.Simulation(dl, dl, dl, 0.9)
+    s.addObject(S.Object("domain", S.Cube(S.Vector(-INF, -INF, 0.0), S.Vector(INF, INF, nz * dl)),
+                         S.Material.createAir()))
+    lo = round(0.5 * nz) * dl
+    s.addObject(S.Object("slab", S.Cube(S.Vector(-INF, -INF, lo), S.Vector(INF, INF, 0.2 * nz * dl)),
+                         S.Material("m", S.ElectroMagneticProperty(3.0, 1.0, 0.02, 0.0))))
+    s.addWaveformSource(S.TFSF1D(tfsf, True, S.Waveform.gaussian(20e-12, 60e-12)))
+    for f in faces:
+        s.addBoundary(S.PML(pml, f))
+    for q, (at, comp) in enumerate(((1, "EX"), (nz // 2, "HY"), (nz - 2, "EX"))):
+        cell = S.Cube(S.Vector(-INF, -INF, at * dl), S.Vector(INF, INF, dl))
+        s.addMonitor(S.FieldTimeMonitor(f"p{q}", cell, "", comp))
+    s.addMonitor(S.MovieMonitor(S.FieldMonitor(S.Cube(S.Vector(-INF, -INF, 0.0), S.Vector(INF, INF, nz * dl)), "EX"),
+                                7, "movie", ""))
+    return s.spec()
+
+
+# 64, 1024, 2048 and 4096 nodes are the edges of the work-items and their
+# cells; a TFSF face in a CPML layer keeps the separate launches
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+@pytest.mark.parametrize("nz,tfsf,faces", [(30, 12, ("ZN", "ZP")), (47, 5, ("ZP", "ZN")), (48, 12, ("ZP",)),
+                                           (1008, 20, ("ZN", "ZP")), (2031, 12, ("ZN", "ZP")),
+                                           (4080, 12, ("ZN", "ZP")), (8000, 12, ("ZN", "ZP")), (200, 6, ())])
+def test_line_steps_match_separate_launches(monkeypatch, nz, tfsf, faces, precision):
+    spec, steps = _line(nz, tfsf, faces=faces), 260
+    sims = []
+    for on in (True, False):
+        if on:
+            monkeypatch.delenv("XFD_STEP_FUSED", raising=False)
+        else:
+            monkeypatch.setenv("XFD_STEP_FUSED", "0")
+        sim = native.Simulation(spec, precision)
+        sim.init(steps)
+        sim.set_profiling(True)
+        for t0, t1 in ((0, 1), (1, 150), (150, steps)):
+            sim.advance(t0, t1 - t0)
+        assert (sim.kernel_stats()["update_h"][0] == 0) == (on and (tfsf > 8 or not faces))
+        sim.finish()
+        sims.append(sim)
+    a, b = sims
+    # FP32: at most 8 roundings of 6e-8 a step in each run, relative to the
+    # incident wave (1 V/m), whose parts cancel outside the TFSF region
+    tol = 0 if precision == "f64" else 2 * steps * 8 * 6e-8
+    for f in ("EX", "EY", "EZ", "HX", "HY", "HZ"):
+        x, y = a.field(f), b.field(f)
+        assert np.abs(x - y).max() <= tol * (1 if f[0] == "E" else 1 / 376), f
+    for m in range(a.monitor_count()):
+        for x, y in zip(a.monitor_records(m), b.monitor_records(m)):
+            assert np.abs(x - y).max() <= tol * (1 / 376 if m == 1 else 1), m
+    assert np.abs(b.field("EX")).max() > 0

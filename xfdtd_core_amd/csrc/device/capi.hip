@@ -20,6 +20,7 @@
 #include "batch_kernels.hpp"
 #include "half_step.hpp"
 #include "kernels.hpp"
+#include "line_kernels.hpp"
 #include "step_kernels.hpp"
 
 namespace {
@@ -326,6 +327,11 @@ struct xfd_ctx {
   // the far planes i = nx, j = ny, k = nz hold zeros, which their slab
   // corrections keep (they draw on each other only), so no launch visits them
   bool far_zero = true;
+  // 1D: many steps per launch (k_line); the record and probe lists above are
+  // then by work-item
+  bool line = false;
+  int line_threads = 0, line_extra_e = 0, line_extra_h = 0;
+  DevBuf loc_e, loc_h, line_extra, line_add_e, line_add_h;
   DevBuf half_e, half_h;  // HalfSlabs of each half-step
   DevBuf rec_off_e, seg_of_e, rec_off_h, seg_of_h, probe_off, probe_of;
   int parity = 0;
@@ -696,6 +702,83 @@ bool slabsByAxis(const xfd_ctx& c, int n[3], int slab[3][2], int swap[3]) {
   return true;
 }
 
+// Items by bin: bin b owns of[off[b] .. off[b + 1]), in item order.
+template <class F>
+void listByBin(int64_t bins, size_t count, F&& bin, DevBuf& off, DevBuf& of) {
+  if (count == 0) return;
+  require(count < (size_t{1} << 31), "too many corrections");
+  std::vector<int32_t> o(static_cast<size_t>(bins) + 1, 0), at(count), list(count);
+  for (size_t q = 0; q < count; ++q) {
+    at[q] = static_cast<int32_t>(bin(q));
+    ++o[at[q] + 1];
+  }
+  for (int64_t b = 0; b < bins; ++b) o[b + 1] += o[b];
+  std::vector<int32_t> next(o.begin(), o.end() - 1);
+  for (size_t q = 0; q < count; ++q) list[next[at[q]]++] = static_cast<int32_t>(q);
+  uploadVector(o, off);
+  uploadVector(list, of);
+}
+
+// Chooses the 1D kernel that steps many times in one launch (k_line): every
+// correction on Ex or Hy of the column (0, 0), or of (0, 1) away from the CPML
+// layers (a TFSF face corrects both), every probe one of those two,
+// no line recordings, and a line that fits one work-group's LDS.
+// XFD_STEP_FUSED=0 keeps a launch per correction.
+void lineSetup(xfd_ctx& c, const std::vector<xfd::Record>& re, const std::vector<int64_t>& se,
+               const std::vector<xfd::Record>& rh, const std::vector<int64_t>& sh,
+               const std::vector<xfd::Probe>& probes) {
+  const char* env = std::getenv("XFD_STEP_FUSED");
+  if (c.dim != 1 || c.n_line > 0 || (env && env[0] == '0') || c.slabs.size() > 2) return;
+  // a correction in the column (0, 1) has no CPML layer next to it
+  auto inReach = [&](bool is_e, int64_t k) {
+    for (const auto& s : c.slabs)
+      if (is_e ? (k >= s->h_start && k <= s->h_start + s->n) : (k >= s->e_start - 1 && k < s->e_start + s->n))
+        return true;
+    return false;
+  };
+  int extra[2] = {0, 0};
+  std::vector<int32_t> loc[2], extra_cell;
+  for (int is_e = 0; is_e < 2; ++is_e) {
+    const auto& rec = is_e ? re : rh;
+    const auto& seg = is_e ? se : sh;
+    for (int64_t q = 0; q < (is_e ? c.nseg_e : c.nseg_h); ++q) {
+      const auto& r = rec[seg[q]];
+      const int64_t column = r.target / c.g.pz, k = r.target % c.g.pz;
+      if (r.field != (is_e ? 0 : 4) || column > 1 || (column == 1 && inReach(is_e != 0, k))) return;
+      if (is_e && column) extra_cell.push_back(static_cast<int32_t>(k));
+      loc[is_e].push_back(static_cast<int32_t>(column ? c.g.nz + 1 + extra[is_e]++ : k));
+    }
+  }
+  if (extra[0] > xfd::kLineExtra || extra[1] > xfd::kLineExtra) return;
+  for (const auto& p : probes)
+    if ((p.field != 0 && p.field != 4) || p.idx > c.g.nz) return;
+  int slab_cells = 0;
+  for (const auto& s : c.slabs) slab_cells += s->n;
+  const int held = static_cast<int>((c.nseg_e <= xfd::kLineSegments ? c.nseg_e : 0) +
+                                    (c.nseg_h <= xfd::kLineSegments ? c.nseg_h : 0));
+  const size_t lds = c.elem == 8 ? xfd::LineLaunch<double>::ldsBytes(c.g.nz, extra[0] + extra[1], slab_cells, held)
+                                 : xfd::LineLaunch<float>::ldsBytes(c.g.nz, extra[0] + extra[1], slab_cells, held);
+  if (slab_cells > xfd::kLineSlabCells || c.g.nz + 1 > xfd::kLineThreads * xfd::kLineCells ||
+      lds > (size_t{160} << 10))
+    return;
+  c.line = true;
+  c.line_extra_e = extra[1];
+  c.line_extra_h = extra[0];
+  if (c.nseg_e <= xfd::kLineSegments) c.line_add_e.alloc(c.nseg_e * xfd::kLineSteps * sizeof(double));
+  if (c.nseg_h <= xfd::kLineSegments) c.line_add_h.alloc(c.nseg_h * xfd::kLineSteps * sizeof(double));
+  uploadVector(loc[1], c.loc_e);
+  uploadVector(loc[0], c.loc_h);
+  c.line_threads = static_cast<int>(std::min<int64_t>(xfd::kLineThreads, (c.g.nz + 64) / 64 * 64));
+  uploadVector(extra_cell, c.line_extra);
+  // a column's correction goes to the cell's work-item; the other column's to
+  // one of the next wavefront, so the two run side by side
+  const int64_t w = c.line_threads;
+  auto owner = [&](const xfd::Record& r) { return (r.target % c.g.pz + r.target / c.g.pz * 64) % w; };
+  listByBin(w, static_cast<size_t>(c.nseg_e), [&](size_t q) { return owner(re[se[q]]); }, c.rec_off_e, c.seg_of_e);
+  listByBin(w, static_cast<size_t>(c.nseg_h), [&](size_t q) { return owner(rh[sh[q]]); }, c.rec_off_h, c.seg_of_h);
+  listByBin(w, probes.size(), [&](size_t q) { return probes[q].idx % w; }, c.probe_off, c.probe_of);
+}
+
 // Chooses the one-launch half-step (k_half) and lists its records and probes
 // by tile.  It takes every 3D grid but those where the order of corrections
 // would differ (a record on a point that a slab corrects, slabs that share
@@ -740,26 +823,15 @@ void halfSetup(xfd_ctx& c, const std::vector<xfd::Record>& re, const std::vector
   const int64_t nbx = (g.nz + c.half_tk - 1) / c.half_tk, nby = (g.ny + c.half_tj - 1) / c.half_tj;
   const int64_t tiles = nbx * nby * ((g.nx + c.half_chunk - 1) / c.half_chunk);
   require(tiles < (int64_t{1} << 31), "grid too large");
-  auto byTile = [&](size_t count, auto&& target, DevBuf& off, DevBuf& of) {
-    if (count == 0) return;
-    require(count < (size_t{1} << 31), "too many corrections");
-    std::vector<int32_t> o(static_cast<size_t>(tiles) + 1, 0), at(count), list(count);
-    for (size_t q = 0; q < count; ++q) {
-      const int64_t x = target(q), rem = x % g.plane;
-      const int64_t i = std::min<int64_t>(x / g.plane, g.nx - 1), j = std::min<int64_t>(rem / g.pz, g.ny - 1),
-                    k = std::min<int64_t>(rem % g.pz, g.nz - 1);
-      at[q] = static_cast<int32_t>((i / c.half_chunk * nby + j / c.half_tj) * nbx + k / c.half_tk);
-      ++o[at[q] + 1];
-    }
-    for (int64_t b = 0; b < tiles; ++b) o[b + 1] += o[b];
-    std::vector<int32_t> next(o.begin(), o.end() - 1);
-    for (size_t q = 0; q < count; ++q) list[next[at[q]]++] = static_cast<int32_t>(q);
-    uploadVector(o, off);
-    uploadVector(list, of);
+  auto tile = [&](int64_t x) {  // a probe on a far plane goes to the nearest tile
+    const int64_t rem = x % g.plane;
+    const int64_t i = std::min<int64_t>(x / g.plane, g.nx - 1), j = std::min<int64_t>(rem / g.pz, g.ny - 1),
+                  k = std::min<int64_t>(rem % g.pz, g.nz - 1);
+    return (i / c.half_chunk * nby + j / c.half_tj) * nbx + k / c.half_tk;
   };
-  byTile(static_cast<size_t>(c.nseg_e), [&](size_t q) { return re[se[q]].target; }, c.rec_off_e, c.seg_of_e);
-  byTile(static_cast<size_t>(c.nseg_h), [&](size_t q) { return rh[sh[q]].target; }, c.rec_off_h, c.seg_of_h);
-  byTile(probes.size(), [&](size_t q) { return probes[q].idx; }, c.probe_off, c.probe_of);
+  listByBin(tiles, static_cast<size_t>(c.nseg_e), [&](size_t q) { return tile(re[se[q]].target); }, c.rec_off_e, c.seg_of_e);
+  listByBin(tiles, static_cast<size_t>(c.nseg_h), [&](size_t q) { return tile(rh[sh[q]].target); }, c.rec_off_h, c.seg_of_h);
+  listByBin(tiles, probes.size(), [&](size_t q) { return tile(probes[q].idx); }, c.probe_off, c.probe_of);
 }
 
 template <class T>
@@ -1362,6 +1434,7 @@ void createTyped(xfd_ctx& c, const xfd_desc& d) {
     }
   }
   halfSetup(c, re, se, rh, sh, probes, records_meet_slabs);
+  lineSetup(c, re, se, rh, sh, probes);
   if (c.half) {
     uploadVector(halfSlabs<T>(c, true), c.half_e);
     uploadVector(halfSlabs<T>(c, false), c.half_h);
@@ -1552,6 +1625,44 @@ xfd::HalfArgs<T> halfArgs(xfd_ctx& c, bool is_e, bool probes) {
 }
 
 template <class T>
+xfd::LineArgs<T> lineArgs(xfd_ctx& c, bool probes) {
+  xfd::LineArgs<T> a{};
+  a.nz = c.g.nz;
+  a.threads = c.line_threads;
+  a.extra_cell = c.line_extra.as<int32_t>();
+  a.extra_e = c.line_extra_e;
+  a.extra_h = c.line_extra_h;
+  a.ex = c.fields[0].as<T>();
+  a.hy = c.fields[4].as<T>();
+  a.hz = c.fields[5].as<T>();
+  a.slabs = static_cast<int>(c.slabs.size());
+  for (int q = 0; q < a.slabs; ++q) {  // component A of the E half is Ex, component B of the H half Hy
+    const auto e = slabArgs<T>(*c.slabs[q], true), h = slabArgs<T>(*c.slabs[q], false);
+    a.e[q] = {e.start, e.n, e.cpsiA, e.psiA, e.ca, e.cb};
+    a.h[q] = {h.start, h.n, h.cpsiB, h.psiB, h.ca, h.cb};
+  }
+  auto events = [](int64_t nseg, DevBuf& off, DevBuf& of, DevBuf& loc, DevBuf& rec, DevBuf& seg, DevBuf& add) {
+    xfd::LineEvents<T> e{};
+    if (!nseg) return e;
+    e = {off.as<int32_t>(), of.as<int32_t>(), loc.as<int32_t>(), rec.as<xfd::Record>(), seg.as<int64_t>(), nseg,
+         add.p ? static_cast<int>(nseg) : 0, add.as<double>()};
+    return e;
+  };
+  a.re = events(c.nseg_e, c.rec_off_e, c.seg_of_e, c.loc_e, c.rec_e, c.seg_e, c.line_add_e);
+  a.rh = events(c.nseg_h, c.rec_off_h, c.seg_of_h, c.loc_h, c.rec_h, c.seg_h, c.line_add_h);
+  a.pool = c.pool.as<double>();
+  a.state = c.state.as<T>();
+  if (probes && c.nprobe) {
+    a.probe_off = c.probe_off.as<int32_t>();
+    a.probe_of = c.probe_of.as<int32_t>();
+    a.probe = c.probe_list.as<xfd::Probe>();
+    a.probe_out = c.probe_out.as<double>();
+    a.probe_count = c.probe_count;
+  }
+  return a;
+}
+
+template <class T>
 void stepTyped(xfd_ctx& c, int64_t t0, int64_t n, bool record = true) {
   require(t0 >= 0 && n >= 0, "bad step range");
   require(t0 + n <= c.pool_rows, "step beyond the source tables (run length given at init)");
@@ -1615,6 +1726,56 @@ void stepTyped(xfd_ctx& c, int64_t t0, int64_t n, bool record = true) {
     const int x = a.axis;
     return a.lo[x] + a.ext[x] <= b.lo[x] || b.lo[x] + b.ext[x] <= a.lo[x];
   };
+  auto recordFrames = [&](int64_t t) {
+    for (auto& gp : c.gathers) {
+      const auto& d = gp->d;
+      if (gp->probe >= 0) continue;
+      if (t < d.first || (t - d.first) % d.interval != 0) continue;
+      const int64_t frame = (t - d.first) / d.interval;
+      if (frame >= d.count) continue;
+      if (gp->staged) {
+        const int slot = static_cast<int>(frame & 1);
+        double* ring = gp->out.as<double>() + slot * gp->a.frame_elems;
+        const size_t fb = static_cast<size_t>(gp->a.frame_elems) * sizeof(double);
+        if (frame >= 2) XFD_HIP(hipStreamWaitEvent(st, gp->copied[slot], 0));  // the slot's last copy is done
+        c.timed(K_GATHER, [&] { xfd::Launch<T>::gather(st, c.g, F, gp->a, ring); });
+        XFD_HIP(hipEventRecord(gp->gathered, st));
+        XFD_HIP(hipStreamWaitEvent(c.copy_stream, gp->gathered, 0));
+        XFD_HIP(hipMemcpyAsync(gp->host + frame * gp->a.frame_elems, ring, fb, hipMemcpyDeviceToHost,
+                               c.copy_stream));
+        XFD_HIP(hipEventRecord(gp->copied[slot], c.copy_stream));
+        continue;
+      }
+      c.timed(K_GATHER, [&] {
+        xfd::Launch<T>::gather(st, c.g, F, gp->a, gp->out.as<double>() + frame * gp->a.frame_elems);
+      });
+    }
+  };
+  if (c.line) {
+    // up to the next step that records a frame, or kLineSteps, per launch
+    const auto a = lineArgs<T>(c, record);
+    for (int64_t t = t0; t < t0 + n;) {
+      int64_t stop = std::min(t0 + n, t + xfd::kLineSteps);
+      for (auto& gp : c.gathers) {
+        if (gp->probe >= 0 || !record) continue;
+        const auto& d = gp->d;
+        const int64_t frame = t <= d.first ? 0 : (t - d.first + d.interval - 1) / d.interval;
+        if (frame < d.count) stop = std::min(stop, std::max(t, d.first + frame * d.interval) + 1);
+      }
+      c.timed(K_STEP, [&] {
+        if (c.classed)
+          xfd::LineLaunch<T>::steps(st, K, a, t, stop - t);
+        else
+          xfd::LineLaunch<T>::steps(st, C, a, t, stop - t);
+      });
+      if (record) recordFrames(stop - 1);
+      t = stop;
+    }
+    XFD_HIP(hipGetLastError());
+    XFD_HIP(hipStreamSynchronize(st));
+    if (c.prof) c.drainEvents();
+    return;
+  }
   for (int64_t t = t0; t < t0 + n; ++t) {
     if (c.fstep) {
       // H, its CPML, E and its CPML in one pass from the current set into
@@ -1712,29 +1873,7 @@ void stepTyped(xfd_ctx& c, int64_t t0, int64_t n, bool record = true) {
         xfd::Launch<T>::probes(st, F, c.probe_list.as<xfd::Probe>(), c.nprobe, c.probe_out.as<double>(),
                                c.probe_count, t);
       });
-    for (auto& gp : c.gathers) {
-      const auto& d = gp->d;
-      if (gp->probe >= 0) continue;
-      if (t < d.first || (t - d.first) % d.interval != 0) continue;
-      const int64_t frame = (t - d.first) / d.interval;
-      if (frame >= d.count) continue;
-      if (gp->staged) {
-        const int slot = static_cast<int>(frame & 1);
-        double* ring = gp->out.as<double>() + slot * gp->a.frame_elems;
-        const size_t fb = static_cast<size_t>(gp->a.frame_elems) * sizeof(double);
-        if (frame >= 2) XFD_HIP(hipStreamWaitEvent(st, gp->copied[slot], 0));  // the slot's last copy is done
-        c.timed(K_GATHER, [&] { xfd::Launch<T>::gather(st, c.g, F, gp->a, ring); });
-        XFD_HIP(hipEventRecord(gp->gathered, st));
-        XFD_HIP(hipStreamWaitEvent(c.copy_stream, gp->gathered, 0));
-        XFD_HIP(hipMemcpyAsync(gp->host + frame * gp->a.frame_elems, ring, fb, hipMemcpyDeviceToHost,
-                               c.copy_stream));
-        XFD_HIP(hipEventRecord(gp->copied[slot], c.copy_stream));
-        continue;
-      }
-      c.timed(K_GATHER, [&] {
-        xfd::Launch<T>::gather(st, c.g, F, gp->a, gp->out.as<double>() + frame * gp->a.frame_elems);
-      });
-    }
+    recordFrames(t);
     if (c.n_line && t < c.line_count)
       c.timed(K_GATHER, [&] {
         xfd::Launch<T>::lines(st, F, c.line_terms.as<xfd::LineTerm>(), c.line_off.as<int64_t>(),
@@ -2519,6 +2658,11 @@ int xfd_write_field(xfd_ctx* c, int32_t field, const double* src) {
   return guard([&] {
     require(c && src && field >= 0 && field < 6, "bad argument");
     if (field == 0 || field == 1 || field == 5) c->te_zero = false;  // no longer known to stay zero
+    if (c->line && field != 5) {  // 1D: what is not Ex or Hy of the column (0, 0) no longer stays zero
+      const int64_t n = field == 0 ? c->g.nz + 1 : c->g.nz;
+      c->line = field == 0 || field == 4;
+      for (int64_t k = n; k < 2 * n && c->line; ++k) c->line = src[k] == 0.0;
+    }
     int ext[3];
     extentOf(field, c->g.nx, c->g.ny, c->g.nz, ext);
     if (c->half && c->far_zero) {  // a far plane that no longer holds zeros takes its slab corrections

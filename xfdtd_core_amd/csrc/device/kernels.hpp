@@ -960,15 +960,9 @@ __global__ __launch_bounds__(256) void k_far_reduce(int na, int chunks, const do
 // that cell's records in the reference's corrector order.  `state` holds the
 // inductor currents (one slot per inductor edge).
 template <class T>
-__device__ __forceinline__ void recordSeg(const FieldPtrs<T>& F, const Record* __restrict__ rec,
-                                          const int64_t* __restrict__ seg, int64_t nseg,
-                                          const double* __restrict__ pool, T* __restrict__ state, int64_t s,
-                                          int64_t t) {
-  if (s >= nseg) return;
-  const int64_t r0 = seg[s], r1 = seg[s + 1];
-  T* f = F.f[rec[r0].field];
-  const int64_t target = rec[r0].target;
-  double acc = static_cast<double>(f[target]);
+__device__ __forceinline__ T recordRun(T value, const Record* __restrict__ rec, int64_t r0, int64_t r1,
+                                       const double* __restrict__ pool, T* __restrict__ state, int64_t t) {
+  double acc = static_cast<double>(value);
   for (int64_t r = r0; r < r1; ++r) {
     const Record R = rec[r];
     if (R.kind == 0) {
@@ -989,7 +983,19 @@ __device__ __forceinline__ void recordSeg(const FieldPtrs<T>& F, const Record* _
     }
     if (sizeof(T) == sizeof(float)) acc = static_cast<double>(static_cast<T>(acc));
   }
-  f[target] = static_cast<T>(acc);
+  return static_cast<T>(acc);
+}
+
+template <class T>
+__device__ __forceinline__ void recordSeg(const FieldPtrs<T>& F, const Record* __restrict__ rec,
+                                          const int64_t* __restrict__ seg, int64_t nseg,
+                                          const double* __restrict__ pool, T* __restrict__ state, int64_t s,
+                                          int64_t t) {
+  if (s >= nseg) return;
+  const int64_t r0 = seg[s], r1 = seg[s + 1];
+  T* f = F.f[rec[r0].field];
+  const int64_t target = rec[r0].target;
+  f[target] = recordRun<T>(f[target], rec, r0, r1, pool, state, t);
 }
 
 template <class T>

@@ -7,3 +7,4 @@ template struct xfd::BatchLaunch<float>;
 template struct xfd::AdjLaunch<float>;
 template struct xfd::StepLaunch<float>;
 template struct xfd::HalfLaunch<float>;
+template struct xfd::LineLaunch<float>;

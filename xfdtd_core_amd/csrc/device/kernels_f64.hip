@@ -7,3 +7,4 @@ template struct xfd::BatchLaunch<double>;
 template struct xfd::AdjLaunch<double>;
 template struct xfd::StepLaunch<double>;
 template struct xfd::HalfLaunch<double>;
+template struct xfd::LineLaunch<double>;

@@ -10,6 +10,7 @@
 #include "batch_kernels.hpp"
 #include "half_step.hpp"
 #include "kernels.hpp"
+#include "line_kernels.hpp"
 #include "step_kernels.hpp"
 
 namespace xfd {
@@ -576,6 +577,41 @@ template <class T>
 void HalfLaunch<T>::half(hipStream_t s, const Grid& g, const FieldPtrs<T>& F, const WideCoef<T>& C,
                          const HalfArgs<T>& a, bool is_e, int64_t t) {
   launchHalfTile<T>(s, g, F, C, a, is_e, t);
+}
+
+template <class T, class Coef, int C>
+void launchLine(hipStream_t s, const Coef& K, const LineArgs<T>& a, int64_t t0, int64_t n) {
+  const size_t lds = LineLaunch<T>::ldsBytes(a.nz, a.extra_e + a.extra_h,
+                                             (a.slabs > 0 ? a.e[0].n : 0) + (a.slabs > 1 ? a.e[1].n : 0),
+                                             a.re.held + a.rh.held);
+  if (lds > (size_t(64) << 10))  // the default limit of dynamic LDS
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_line<T, Coef, C>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+  for (const auto* e : {&a.re, &a.rh})
+    if (e->addends)
+      hipLaunchKernelGGL(k_line_addends<T>, dim3(blocks_for(n, 256), static_cast<unsigned>(e->nseg)), dim3(256), 0, s,
+                         e->rec, e->seg, e->nseg, a.pool, t0, n, e->addends);
+  hipLaunchKernelGGL((k_line<T, Coef, C>), dim3(1), dim3(a.threads), lds, s, K, a, t0, static_cast<int>(n));
+}
+template <class T, class Coef>
+void launchLineCells(hipStream_t s, const Coef& K, const LineArgs<T>& a, int64_t t0, int64_t n) {
+  const int c = (a.nz + a.threads) / a.threads;  // cells per work-item: nz + 1 over the work-items
+  if (c <= 1)
+    launchLine<T, Coef, 1>(s, K, a, t0, n);
+  else if (c <= 2)
+    launchLine<T, Coef, 2>(s, K, a, t0, n);
+  else if (c <= 4)
+    launchLine<T, Coef, 4>(s, K, a, t0, n);
+  else
+    launchLine<T, Coef, kLineCells>(s, K, a, t0, n);
+}
+template <class T>
+void LineLaunch<T>::steps(hipStream_t s, const CoefPtrs<T>& C, const LineArgs<T>& a, int64_t t0, int64_t n) {
+  launchLineCells<T>(s, C, a, t0, n);
+}
+template <class T>
+void LineLaunch<T>::steps(hipStream_t s, const ClassCoef<T>& C, const LineArgs<T>& a, int64_t t0, int64_t n) {
+  launchLineCells<T>(s, C, a, t0, n);
 }
 
 }  // namespace xfd
