@@ -127,3 +127,68 @@ def test_half_step_far_planes(monkeypatch):
         runs.append(sim)
     _compare(*runs, "f64", "far planes")
     assert np.abs(runs[0].field("EX")[:, :, -1]).max() > 0
+
+
+def _plane(nx, ny, faces=("XN", "XP", "YN", "YP"), pml=6, tfsf=12):
+    """A 2D grid of nx x ny cells including the CPML: a lossy cylinder in a
+    plane wave, probes and a movie."""
+    inf, dl = float("inf"), 1e-3
+    inner = [nx - sum(pml for f in faces if f[0] == "X"), ny - sum(pml for f in faces if f[0] == "Y")]
+    s = S.Simulation(dl, dl, 1.0, 0.9)
+    size = [m * dl for m in inner]
+    s.addObject(S.Object("domain", S.Cube(S.Vector(0, 0, -inf), S.Vector(*size, inf)), S.Material.createAir()))
+    s.addObject(S.Object("rod", S.Cylinder(S.Vector(size[0] / 2, size[1] / 2, -inf), 4 * dl, inf, "Z"),
+                         S.Material("m", S.ElectroMagneticProperty(3.0, 1.0, 0.02, 0.0))))
+    s.addWaveformSource(S.TFSF2D(tfsf, tfsf, 0.6, S.Waveform.gaussian(20e-12, 60e-12)))
+    for f in faces:
+        s.addBoundary(S.PML(pml, f))
+    for q, (at, comp) in enumerate((((1, 1), "EZ"), ((inner[0] // 2, inner[1] // 2), "HX"),
+                                    ((inner[0] - 1, inner[1] - 1), "EZ"))):
+        s.addMonitor(S.FieldTimeMonitor(f"p{q}", S.Cube(S.Vector(at[0] * dl, at[1] * dl, -inf), S.Vector(dl, dl, inf)),
+                                        "", comp))
+    s.addMonitor(S.MovieMonitor(S.FieldMonitor(S.Cube(S.Vector(0, 0, -inf), S.Vector(*size, inf)), "EZ"), 9, "movie",
+                                ""))
+    return s.spec()
+
+
+# ny around the 64 lanes, nx around the 4 wavefronts and their rows, slab orders
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+@pytest.mark.parametrize("nx,ny,chunk,faces", [(37, 63, None, ("XN", "XP", "YN", "YP")),
+                                               (33, 65, 3, ("YP", "YN", "XP", "XN")), (40, 128, 16, ("YN", "XP")),
+                                               (64, 33, 1, ())])
+def test_plane_half_step(monkeypatch, nx, ny, chunk, faces, precision):
+    spec, steps = _plane(nx, ny, faces), 120
+    runs = []
+    for on in (True, False):
+        sim = _run(monkeypatch, spec, precision, steps, on, chunk)
+        sim.advance(0, 50)
+        sim.advance(50, steps - 50)
+        sim.finish()
+        runs.append(sim)
+    a, b = runs
+    # FP32 as above, relative to the incident wave (1 V/m)
+    tol = 0 if precision == "f64" else 2 * steps * 8 * 6e-8
+    for f in FIELDS:
+        assert np.abs(a.field(f) - b.field(f)).max() <= tol * (1 if f[0] == "E" else 1 / 376), f
+    for m in range(a.monitor_count()):
+        for x, y in zip(a.monitor_records(m), b.monitor_records(m)):
+            assert np.abs(x - y).max() <= tol * (1 / 376 if m == 1 else 1), m
+    assert np.abs(b.field("EZ")).max() > 0
+
+
+def test_plane_half_step_after_writes(monkeypatch):
+    """A field that no longer stays zero takes a 2D grid off the one launch."""
+    spec, steps = _plane(40, 44), 40
+    runs = []
+    for on in (True, False):
+        sim = _run(monkeypatch, spec, "f64", steps, on)
+        sim.advance(0, 10)
+        rng = np.random.default_rng(5)
+        for q, ext in ((2, (41, 45, 1)), (5, (40, 44, 2))):
+            v = np.ascontiguousarray(rng.standard_normal(ext))
+            assert native.load_library().xfd_write_field(ctypes.c_void_p(sim.device_context()), q, v.ctypes.data) == 0
+        sim.advance(10, steps - 10)
+        sim.finish()
+        runs.append(sim)
+    _te = [np.abs(runs[0].field(f) - runs[1].field(f)).max() for f in FIELDS]
+    assert _te == [0] * 6

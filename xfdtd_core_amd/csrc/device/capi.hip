@@ -22,6 +22,7 @@
 #include "kernels.hpp"
 #include "line_kernels.hpp"
 #include "step_kernels.hpp"
+#include "te_kernels.hpp"
 
 namespace {
 
@@ -166,7 +167,7 @@ bool classify(const double* A, const double* B, const double* C, const int ext[3
               last_id = id.at(t);
               have = true;
             }
-            ids[(i * g.NY + j) * g.pz + k] = last_id;
+            ids[g.at(i, j, k)] = last_id;
           }
     });
   for (auto& t : th) t.join();
@@ -520,7 +521,7 @@ void uploadVector(const std::vector<T>& v, DevBuf& b) {
   if (!v.empty()) XFD_HIP(hipMemcpy(b.p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
 }
 
-int64_t padIndex(const xfd::Grid& g, int64_t i, int64_t j, int64_t k) { return (i * g.NY + j) * g.pz + k; }
+int64_t padIndex(const xfd::Grid& g, int64_t i, int64_t j, int64_t k) { return g.at(i, j, k); }
 
 // Expands the TFSF corrector loops (tfsf_corrector.h:89-229, call order
 // tfsf_corrector.cpp:177-232) into per-cell records for one half-step.
@@ -649,8 +650,8 @@ void segment(std::vector<xfd::Record>& rec, std::vector<int64_t>& seg) {
 // separate CPML launches.
 bool recordsMeetSlabs(const xfd_ctx& c, const std::vector<xfd::Record>& recs, bool is_e) {
   for (const auto& r : recs) {
-    const int64_t i = r.target / c.g.plane, rem = r.target % c.g.plane;
-    const int64_t p[3] = {i, rem / c.g.pz, rem % c.g.pz};
+    int64_t p[3];
+    c.g.point(r.target, p);
     for (const auto& sl : c.slabs) {
       const int* lo = is_e ? sl->lo_e : sl->lo_h;
       bool in = true;
@@ -780,7 +781,8 @@ void lineSetup(xfd_ctx& c, const std::vector<xfd::Record>& re, const std::vector
 }
 
 // Chooses the one-launch half-step (k_half) and lists its records and probes
-// by tile.  It takes every 3D grid but those where the order of corrections
+// by tile.  It takes every 3D grid, and every 2D grid whose Ex, Ey
+// and Hz stay zero (k_te_half), but those where the order of corrections
 // would differ (a record on a point that a slab corrects, slabs that share
 // planes or interleave their axes) and those with a record on a far plane,
 // which no tile visits.  XFD_CPML_INSWEEP=0 and XFD_STEP_FUSED=0 keep a launch
@@ -796,11 +798,12 @@ void halfSetup(xfd_ctx& c, const std::vector<xfd::Record>& re, const std::vector
   bool far = false;
   for (const auto* v : {&re, &rh})
     for (const auto& r : *v) {
-      const int64_t rem = r.target % g.plane;
-      far = far || r.target / g.plane >= g.nx || rem / g.pz >= g.ny || rem % g.pz >= g.nz;
+      int64_t p[3];
+      g.point(r.target, p);
+      far = far || p[0] >= g.nx || p[1] >= g.ny || p[2] >= g.nz;
     }
   int n[3], slab[3][2], swap[3];
-  c.half = c.dim == 3 && !c.fstep && !records_meet_slabs && !far && slabsByAxis(c, n, slab, swap) &&
+  c.half = (c.dim == 3 || (c.dim == 2 && c.te_zero)) && !c.fstep && !records_meet_slabs && !far && slabsByAxis(c, n, slab, swap) &&
            !is("XFD_CPML_INSWEEP", '0') && !is("XFD_STEP_FUSED", '0') && !is("XFD_CPML_FUSED", '1') &&
            !is("XFD_CPML_ZFUSED", '1');
   if (!c.half) return;
@@ -808,7 +811,7 @@ void halfSetup(xfd_ctx& c, const std::vector<xfd::Record>& re, const std::vector
   c.n_fused = 0;
   c.zfused = false;
   std::fill(c.zslab.begin(), c.zslab.end(), 0);
-  if (xfd::sweepTile128(g)) {
+  if (c.dim == 3 && xfd::sweepTile128(g)) {
     c.half_tk = 128;
     c.half_tj = 2;
   }
@@ -820,13 +823,22 @@ void halfSetup(xfd_ctx& c, const std::vector<xfd::Record>& re, const std::vector
     const int64_t rows = ((g.nz + 63) / 64) * ((g.ny + 3) / 4);
     c.half_chunk = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(4, g.nx * rows / 1024)));
   }
-  const int64_t nbx = (g.nz + c.half_tk - 1) / c.half_tk, nby = (g.ny + c.half_tj - 1) / c.half_tj;
-  const int64_t tiles = nbx * nby * ((g.nx + c.half_chunk - 1) / c.half_chunk);
+  int64_t nbx = (g.nz + c.half_tk - 1) / c.half_tk, nby = (g.ny + c.half_tj - 1) / c.half_tj;
+  int64_t tiles = nbx * nby * ((g.nx + c.half_chunk - 1) / c.half_chunk);
+  if (c.dim == 2) {  // 64 points of a row per wavefront, a march of rows each
+    nbx = (g.ny + 63) / 64;
+    if (!std::getenv("XFD_ICHUNK"))
+      c.half_chunk = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(4, g.nx * nbx / 8192)));
+    const int64_t rows = static_cast<int64_t>(xfd::kTeRows) * c.half_chunk;
+    tiles = nbx * ((g.nx + rows - 1) / rows);
+  }
   require(tiles < (int64_t{1} << 31), "grid too large");
   auto tile = [&](int64_t x) {  // a probe on a far plane goes to the nearest tile
-    const int64_t rem = x % g.plane;
-    const int64_t i = std::min<int64_t>(x / g.plane, g.nx - 1), j = std::min<int64_t>(rem / g.pz, g.ny - 1),
-                  k = std::min<int64_t>(rem % g.pz, g.nz - 1);
+    int64_t p[3];
+    g.point(x, p);
+    const int64_t i = std::min<int64_t>(p[0], g.nx - 1), j = std::min<int64_t>(p[1], g.ny - 1),
+                  k = std::min<int64_t>(p[2], g.nz - 1);
+    if (c.dim == 2) return i / (xfd::kTeRows * c.half_chunk) * nbx + j / 64;
     return (i / c.half_chunk * nby + j / c.half_tj) * nbx + k / c.half_tk;
   };
   listByBin(tiles, static_cast<size_t>(c.nseg_e), [&](size_t q) { return tile(re[se[q]].target); }, c.rec_off_e, c.seg_of_e);
@@ -1702,7 +1714,11 @@ void stepTyped(xfd_ctx& c, int64_t t0, int64_t n, bool record = true) {
   auto half = [&](bool is_e, int64_t t) {
     const auto& a = is_e ? HE : HH;
     c.timed(is_e ? K_UPDATE_E : K_UPDATE_H, [&] {
-      if (c.wide)
+      if (c.dim == 2 && c.classed)
+        xfd::TeLaunch<T>::half(st, c.g, F, K, a, is_e, t);
+      else if (c.dim == 2)
+        xfd::TeLaunch<T>::half(st, c.g, F, C, a, is_e, t);
+      else if (c.wide)
         xfd::HalfLaunch<T>::half(st, c.g, F, M, a, is_e, t);
       else if (c.classed)
         xfd::HalfLaunch<T>::half(st, c.g, F, K, a, is_e, t);
@@ -2600,11 +2616,16 @@ int xfd_create(const xfd_desc* d, xfd_ctx** out) {
     g.nz = d->nz;
     g.NY = d->ny + 1;
     const int64_t line = 128 / static_cast<int64_t>(c->elem);
-    // a 2D grid keeps k's two entries unpadded, so its rows along j are
-    // contiguous (pitch 2) for the TE kernels' lanes
-    g.pz = dim == 2 ? 2 : ((d->nz + 1) + line - 1) / line * line;
+    g.pz = ((d->nz + 1) + line - 1) / line * line;
     g.plane = static_cast<int64_t>(g.NY) * g.pz;
     g.total = static_cast<int64_t>(d->nx + 1) * g.plane;
+    g.kz = 1;
+    if (dim == 2) {  // j fastest, k's two entries as two planes
+      g.pz = 1;
+      g.plane = (g.NY + line - 1) / line * line;
+      g.kz = static_cast<int64_t>(d->nx + 1) * g.plane;
+      g.total = 2 * g.kz;
+    }
     const int64_t bxy = ((g.nz + xfd::kLanesK - 1) / xfd::kLanesK) * ((g.ny + xfd::kRowsJ - 1) / xfd::kRowsJ);
     // i-planes marched per sweep work-item: measured on the 384^3 box (FP32 /
     // FP64 ms per step) 1: 1.405 / 2.403, 2: 1.336 / 2.376, 3: 1.324 / 2.373,
@@ -2674,6 +2695,8 @@ int xfd_write_field(xfd_ctx* c, int32_t field, const double* src) {
           for (int k = i == n[0] || j == n[1] ? 0 : n[2]; k < ext[2]; ++k) zero = zero && row[k] == 0.0;
         }
       c->far_zero = zero;
+      // 2D: k_te_half moves k = 0 of Ez, Hx and Hy alone
+      if (c->dim == 2 && !(c->te_zero && zero)) c->half = false;
     }
     DevBuf tmp;
     tmp.alloc(static_cast<size_t>(ext[0]) * ext[1] * ext[2] * sizeof(double));

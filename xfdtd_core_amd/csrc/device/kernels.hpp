@@ -355,9 +355,8 @@ __global__ __launch_bounds__(TK * TJ) void k_update_e(Grid g, FieldPtrs<T> F, Co
   sweepE<T, Coef, Fused, ZF, TK, TJ>(g, F, C, bx, by, bz, ichunk, P, Z);
 }
 
-// 2D (TE) grid, nz = 1, in a layout of pitch pz = 2 along k (k = 1 holds
-// the far face of Ex, Ey and Hz): lanes run along j, the contiguous axis
-// once k has two entries, and work-group rows along i.
+// 2D (TE) grid, nz = 1 (k = 1 holds the far face of Ex, Ey and Hz): lanes run
+// along j, the contiguous axis of its layout, and work-group rows along i.
 //
 // BasicUpdator::updateH (src/updator/basic_updator.cpp:23-41) over
 // [0,nx) x [0,ny) x {0}: all three components with every term, as the
@@ -371,7 +370,7 @@ __global__ __launch_bounds__(256) void k_te_h(Grid g, FieldPtrs<T> F, Coef C) {
   const int i = blockIdx.y * 4 + threadIdx.y;
   if (j >= g.ny || i >= g.nx) return;
   const int64_t pz = g.pz, pl = g.plane;
-  const int64_t idx = (static_cast<int64_t>(i) * g.NY + j) * pz;
+  const int64_t idx = g.at(i, j, 0);
   const T* __restrict__ ex = F.f[0];
   const T* __restrict__ ey = F.f[1];
   const T* __restrict__ ez = F.f[2];
@@ -387,9 +386,9 @@ __global__ __launch_bounds__(256) void k_te_h(Grid g, FieldPtrs<T> F, Coef C) {
     return;
   }
   C.get(3, idx, s, a, b);
-  const T vx = s * F.f[3][idx] + a * (ey[idx + 1] - ey[idx]) + b * (ez[idx + pz] - ez[idx]);
+  const T vx = s * F.f[3][idx] + a * (ey[idx + g.kz] - ey[idx]) + b * (ez[idx + pz] - ez[idx]);
   C.get(4, idx, s, a, b);
-  const T vy = s * F.f[4][idx] + a * (ez[idx + pl] - ez[idx]) + b * (ex[idx + 1] - ex[idx]);
+  const T vy = s * F.f[4][idx] + a * (ez[idx + pl] - ez[idx]) + b * (ex[idx + g.kz] - ex[idx]);
   C.get(5, idx, s, a, b);
   const T vz = s * F.f[5][idx] + a * (ex[idx + pz] - ex[idx]) + b * (ey[idx + pl] - ey[idx]);
   F.f[3][idx] = vx;
@@ -405,7 +404,7 @@ __global__ __launch_bounds__(256) void k_te_e(Grid g, FieldPtrs<T> F, Coef C) {
   const int i = blockIdx.y * 4 + threadIdx.y;
   if (j < 1 || j >= g.ny || i < 1 || i >= g.nx) return;
   const int64_t pz = g.pz, pl = g.plane;
-  const int64_t idx = (static_cast<int64_t>(i) * g.NY + j) * pz;
+  const int64_t idx = g.at(i, j, 0);
   const T* __restrict__ hx = F.f[3];
   const T* __restrict__ hy = F.f[4];
   T s, a, b;
@@ -490,7 +489,7 @@ __device__ __forceinline__ void cpmlPoint(const Grid& g, const FieldPtrs<T>& F, 
   const int c = s.axis, a = c == 2 ? 0 : c + 1, b = c == 0 ? 2 : c - 1;
   const int layer = pick3(c, p0, p1, p2) - s.start;
   const T ca = s.ca[layer], cb = s.cb[layer];
-  const int64_t idx = (static_cast<int64_t>(p0) * g.NY + p1) * g.pz + p2;
+  const int64_t idx = g.at(p0, p1, p2);
   const int64_t q = IsE ? idx - s.stride_c : idx + s.stride_c;
   const int pa = pick3(a, p0, p1, p2), pb = pick3(b, p0, p1, p2);
   if (pa < s.extA[0] && pb < s.extA[1]) {
@@ -1015,7 +1014,7 @@ __global__ __launch_bounds__(256) void k_gather(Grid g, FieldPtrs<T> F, GatherAr
   const int w = static_cast<int>(t % n2);
   const int v = static_cast<int>((t / n2) % n1);
   const int u = static_cast<int>(t / (static_cast<int64_t>(n2) * n1));
-  const int64_t idx = (static_cast<int64_t>(a.o[0] + u) * g.NY + (a.o[1] + v)) * g.pz + (a.o[2] + w);
+  const int64_t idx = g.at(a.o[0] + u, a.o[1] + v, a.o[2] + w);
   out[t] = static_cast<double>(F.f[a.field][idx]);
 }
 
@@ -1030,7 +1029,7 @@ __global__ __launch_bounds__(256) void k_unpack(Grid g, const double* __restrict
   const int w = static_cast<int>(t % n2);
   const int v = static_cast<int>((t / n2) % n1);
   const int u = static_cast<int>(t / (static_cast<int64_t>(n2) * n1));
-  dst[(static_cast<int64_t>(u) * g.NY + v) * g.pz + w] = static_cast<T>(src[t]);
+  dst[g.at(u, v, w)] = static_cast<T>(src[t]);
 }
 
 template <class T>
@@ -1042,7 +1041,7 @@ __global__ __launch_bounds__(256) void k_pack(Grid g, const T* __restrict__ src,
   const int w = static_cast<int>(t % n2);
   const int v = static_cast<int>((t / n2) % n1);
   const int u = static_cast<int>(t / (static_cast<int64_t>(n2) * n1));
-  dst[t] = static_cast<double>(src[(static_cast<int64_t>(u) * g.NY + v) * g.pz + w]);
+  dst[t] = static_cast<double>(src[g.at(u, v, w)]);
 }
 
 // Time-domain NF2FF, phase 1, one thread per (group, cell):

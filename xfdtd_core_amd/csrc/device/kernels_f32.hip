@@ -8,3 +8,4 @@ template struct xfd::AdjLaunch<float>;
 template struct xfd::StepLaunch<float>;
 template struct xfd::HalfLaunch<float>;
 template struct xfd::LineLaunch<float>;
+template struct xfd::TeLaunch<float>;

@@ -8,3 +8,4 @@ template struct xfd::AdjLaunch<double>;
 template struct xfd::StepLaunch<double>;
 template struct xfd::HalfLaunch<double>;
 template struct xfd::LineLaunch<double>;
+template struct xfd::TeLaunch<double>;

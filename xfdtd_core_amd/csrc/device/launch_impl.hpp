@@ -12,6 +12,7 @@
 #include "kernels.hpp"
 #include "line_kernels.hpp"
 #include "step_kernels.hpp"
+#include "te_kernels.hpp"
 
 namespace xfd {
 
@@ -612,6 +613,29 @@ void LineLaunch<T>::steps(hipStream_t s, const CoefPtrs<T>& C, const LineArgs<T>
 template <class T>
 void LineLaunch<T>::steps(hipStream_t s, const ClassCoef<T>& C, const LineArgs<T>& a, int64_t t0, int64_t n) {
   launchLineCells<T>(s, C, a, t0, n);
+}
+
+template <class T, class Coef>
+void launchTeHalf(hipStream_t s, const Grid& g, const FieldPtrs<T>& F, const Coef& C, const HalfArgs<T>& a, bool is_e,
+                  int64_t t) {
+  const unsigned nbx = blocks_for(g.ny, 64), nby = blocks_for(g.nx, kTeRows * a.ichunk);
+  const dim3 grid(nbx * nby), block(64, kTeRows);
+  if (is_e)
+    hipLaunchKernelGGL((k_te_half<T, Coef, true>), grid, block, 0, s, g, F, C, a.slabs, a.events,
+                       static_cast<int>(nbx), a.ichunk, t);
+  else
+    hipLaunchKernelGGL((k_te_half<T, Coef, false>), grid, block, 0, s, g, F, C, a.slabs, a.events,
+                       static_cast<int>(nbx), a.ichunk, t);
+}
+template <class T>
+void TeLaunch<T>::half(hipStream_t s, const Grid& g, const FieldPtrs<T>& F, const CoefPtrs<T>& C,
+                       const HalfArgs<T>& a, bool is_e, int64_t t) {
+  launchTeHalf<T>(s, g, F, C, a, is_e, t);
+}
+template <class T>
+void TeLaunch<T>::half(hipStream_t s, const Grid& g, const FieldPtrs<T>& F, const ClassCoef<T>& C,
+                       const HalfArgs<T>& a, bool is_e, int64_t t) {
+  launchTeHalf<T>(s, g, F, C, a, is_e, t);
 }
 
 }  // namespace xfd

@@ -7,7 +7,9 @@
 // starts on a line boundary and a 64-lane wavefront reading 64 consecutive k
 // touches the minimum number of lines.  A component's own extent (e.g. Ex is
 // nx x (ny+1) x (nz+1)) is a sub-box of the common one; the padding cells are
-// zero and never written.
+// zero and never written.  A 2D grid (nz = 1) has j fastest instead (pz = 1,
+// rows of ny + 1 rounded up to whole lines) and k's two entries as two planes
+// (kz), so that the one that moves is contiguous.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -22,6 +24,17 @@ struct Grid {
   int64_t pz;      // padded k pitch (elements)
   int64_t plane;   // NY * pz
   int64_t total;   // (nx + 1) * plane
+  int64_t kz;      // stride of k: 1, or on a 2D grid one plane of the two
+  __host__ __device__ __forceinline__ int64_t at(int64_t i, int64_t j, int64_t k) const {
+    return i * plane + j * pz + k * kz;
+  }
+  // the point of a padded index
+  __host__ __device__ __forceinline__ void point(int64_t x, int64_t p[3]) const {
+    const int64_t k = kz > 1 ? x / kz : 0, rem = kz > 1 ? x % kz : x;
+    p[0] = rem / plane;
+    p[1] = rem % plane / pz;
+    p[2] = kz > 1 ? k : rem % plane % pz;
+  }
 };
 
 // Work-group order of the Yee sweeps.  The sweep grid is nbx (k) x nby (j)
