@@ -19,6 +19,7 @@
 #include "adjoint_kernels.hpp"
 #include "batch_kernels.hpp"
 #include "half_step.hpp"
+#include "host_stage.hpp"
 #include "kernels.hpp"
 #include "line_kernels.hpp"
 #include "step_kernels.hpp"
@@ -227,6 +228,7 @@ struct DevBuf {
 }  // namespace
 
 struct xfd_ctx {
+  xfd::HostStage::User stage_user;
   int dtype = XFD_F64;
   xfd::Grid g{};
   hipStream_t stream = nullptr;
@@ -346,6 +348,7 @@ struct xfd_ctx {
 
   // checkpoints of a forward run for the adjoint (xfd_forward_checkpointed)
   DevBuf ckpt;
+  DevBuf far_ws;  // xfd_nf2ff_far_field: inputs, partial sums, result
   int64_t ck_interval = 0, ck_nt = 0, ck_bytes = 0;
 
   bool prof = false;
@@ -388,7 +391,7 @@ struct xfd_ctx {
         b += x->bytes;
     for (int q = 0; q < 3; ++q) b += ade_j[q].bytes + ade_jp[q].bytes + ade_eprev[q].bytes;
     for (auto& gth : gathers) b += gth->out.bytes;
-    b += ckpt.bytes;
+    b += ckpt.bytes + far_ws.bytes;
     b += line_terms.bytes + line_off.bytes + line_scale.bytes + line_out.bytes;
     return b;
   }
@@ -507,6 +510,20 @@ xfd::CoefPtrs<T> coefPtrs(xfd_ctx& c) {
 }
 
 // Uploads a double array of the reference extent into a padded device array.
+void checkHip(hipError_t e) { XFD_HIP(e); }
+
+// `count` doubles of device memory to the host.
+void readDoubles(xfd_ctx& c, const double* src, double* dst, size_t count) {
+  xfd::HostStage::read(
+      c.stream, count, sizeof(double), checkHip,
+      [&](size_t first, size_t n, void* slot) {
+        XFD_HIP(hipMemcpyAsync(slot, src + first, n * sizeof(double), hipMemcpyDeviceToHost, c.stream));
+      },
+      [&](size_t first, size_t n, const void* slot) {
+        xfd::HostStage::widen(static_cast<const double*>(slot), dst + first, n);
+      });
+}
+
 template <class T>
 void uploadPadded(xfd_ctx& c, const double* host, const int ext[3], T* dst, DevBuf& staging) {
   const size_t n = static_cast<size_t>(ext[0]) * ext[1] * ext[2];
@@ -2663,15 +2680,24 @@ int xfd_read_field(xfd_ctx* c, int32_t field, double* dst) {
     int ext[3];
     extentOf(field, c->g.nx, c->g.ny, c->g.nz, ext);
     const size_t n = static_cast<size_t>(ext[0]) * ext[1] * ext[2];
-    DevBuf tmp;
-    tmp.alloc(n * sizeof(double));
     DevBuf& cur = curFields(*c)[field];
+    auto read = [&](auto* src) {
+      using T = std::remove_pointer_t<decltype(src)>;
+      xfd::HostStage::read(
+          c->stream, n, sizeof(T), checkHip,
+          [&](size_t first, size_t count, void* slot) {
+            xfd::Launch<T>::pack(c->stream, c->g, src, static_cast<T*>(slot), static_cast<int64_t>(first),
+                                 static_cast<int64_t>(count), ext[1], ext[2]);
+            XFD_HIP(hipGetLastError());
+          },
+          [&](size_t first, size_t count, const void* slot) {
+            xfd::HostStage::widen(static_cast<const T*>(slot), dst + first, count);
+          });
+    };
     if (c->dtype == XFD_F64)
-      xfd::Launch<double>::pack(c->stream, c->g, cur.as<double>(), tmp.as<double>(), ext[0], ext[1], ext[2]);
+      read(cur.as<double>());
     else
-      xfd::Launch<float>::pack(c->stream, c->g, cur.as<float>(), tmp.as<double>(), ext[0], ext[1], ext[2]);
-    XFD_HIP(hipMemcpyAsync(dst, tmp.p, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    XFD_HIP(hipStreamSynchronize(c->stream));
+      read(cur.as<float>());
   });
 }
 
@@ -2724,12 +2750,9 @@ int xfd_read_gather(xfd_ctx* c, int32_t gi, double* dst) {
       return;
     }
     if (g.probe >= 0)
-      XFD_HIP(hipMemcpyAsync(dst, c->probe_out.as<double>() + g.probe * c->probe_count,
-                             static_cast<size_t>(c->probe_count) * sizeof(double), hipMemcpyDeviceToHost,
-                             c->stream));
-    else if (g.out.bytes)
-      XFD_HIP(hipMemcpyAsync(dst, g.out.p, g.out.bytes, hipMemcpyDeviceToHost, c->stream));
-    XFD_HIP(hipStreamSynchronize(c->stream));
+      readDoubles(*c, c->probe_out.as<double>() + g.probe * c->probe_count, dst, static_cast<size_t>(c->probe_count));
+    else
+      readDoubles(*c, g.out.as<double>(), dst, g.out.bytes / sizeof(double));
   });
 }
 
@@ -2800,30 +2823,43 @@ int xfd_nf2ff_far_field(xfd_ctx* c, int32_t n, int32_t f, int32_t na, const doub
     require(na >= 0, "bad direction count");
     if (na == 0) return;
     const int dims[3] = {c->g.nx, c->g.ny, c->g.nz};
-    DevBuf geo[9], ang[2], out;
+    for (int a = 0; a < 3; ++a) require(e_node[a] && h_node[a] && e_size[a], "grid arrays missing");
+    // one upload of everything the kernel reads, into a workspace that grows
+    // to the largest call (eleven allocations and uploads took 0.2 of a call's
+    // 0.33 ms)
+    std::vector<double> in;
     xfd::FarArgs fa{};
+    size_t at[11];
+    auto put = [&](int q, const double* v, int n) {
+      at[q] = in.size();
+      in.insert(in.end(), v, v + n);
+    };
     for (int a = 0; a < 3; ++a) {
-      require(e_node[a] && h_node[a] && e_size[a], "grid arrays missing");
-      uploadVector(std::vector<double>(e_node[a], e_node[a] + dims[a] + 1), geo[a]);
-      uploadVector(std::vector<double>(h_node[a], h_node[a] + dims[a]), geo[3 + a]);
-      uploadVector(std::vector<double>(e_size[a], e_size[a] + dims[a]), geo[6 + a]);
-      fa.e_node[a] = geo[a].as<double>();
-      fa.h_node[a] = geo[3 + a].as<double>();
-      fa.e_size[a] = geo[6 + a].as<double>();
+      put(a, e_node[a], dims[a] + 1);
+      put(3 + a, h_node[a], dims[a]);
+      put(6 + a, e_size[a], dims[a]);
       fa.origin[a] = origin[a];
     }
-    uploadVector(std::vector<double>(theta, theta + na), ang[0]);
-    uploadVector(std::vector<double>(phi, phi + na), ang[1]);
-    fa.theta = ang[0].as<double>();
-    fa.phi = ang[1].as<double>();
+    put(9, theta, na);
+    put(10, phi, na);
     fa.k = k;
-    out.alloc(static_cast<size_t>(na) * 8 * sizeof(double));
-    DevBuf part;
-    part.alloc(static_cast<size_t>(na) * xfd::Launch<double>::farChunks(na) * 8 * sizeof(double));
-    xfd::Launch<double>::far_field(c->stream, N.a, f, fa, na, part.as<double>(), out.as<double>());
+    const size_t n_part = static_cast<size_t>(na) * xfd::Launch<double>::farChunks(na) * 8;
+    const size_t bytes = (in.size() + n_part + static_cast<size_t>(na) * 8) * sizeof(double);
+    if (c->far_ws.bytes < bytes) c->far_ws.alloc(bytes);
+    double* dev = c->far_ws.as<double>();
+    XFD_HIP(hipMemcpyAsync(dev, in.data(), in.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    for (int a = 0; a < 3; ++a) {
+      fa.e_node[a] = dev + at[a];
+      fa.h_node[a] = dev + at[3 + a];
+      fa.e_size[a] = dev + at[6 + a];
+    }
+    fa.theta = dev + at[9];
+    fa.phi = dev + at[10];
+    double* part = dev + in.size();
+    double* out = part + n_part;
+    xfd::Launch<double>::far_field(c->stream, N.a, f, fa, na, part, out);
     XFD_HIP(hipGetLastError());
-    XFD_HIP(hipMemcpyAsync(dst, out.p, out.bytes, hipMemcpyDeviceToHost, c->stream));
-    XFD_HIP(hipStreamSynchronize(c->stream));
+    readDoubles(*c, out, dst, static_cast<size_t>(na) * 8);
   });
 }
 
@@ -3062,9 +3098,7 @@ int xfd_batch_last_ms(xfd_batch* b, double* ms) {
 int xfd_read_line(xfd_ctx* c, int32_t m, double* dst) {
   return guard([&] {
     require(c && dst && m >= 0 && m < c->n_line, "bad line recording index");
-    if (!c->line_count) return;
-    XFD_HIP(hipMemcpy(dst, c->line_out.as<double>() + m * c->line_count, c->line_count * sizeof(double),
-                      hipMemcpyDeviceToHost));
+    readDoubles(*c, c->line_out.as<double>() + m * c->line_count, dst, static_cast<size_t>(c->line_count));
   });
 }
 
@@ -3074,9 +3108,8 @@ int xfd_read_nf2ff(xfd_ctx* c, int32_t n, int32_t f, int32_t d, int32_t which, d
     auto& nn = *c->nf2ffs[n];
     require(f >= 0 && f < nn.a.nf && d >= 0 && d < 6 && which >= 0 && which < 4, "bad NF2FF slice");
     const int64_t cells = nn.a.off[6], cnt = nn.a.off[d + 1] - nn.a.off[d];
-    if (cnt == 0) return;
     const double2* src = nn.acc.as<double2>() + (static_cast<int64_t>(f) * 4 + which) * cells + nn.a.off[d];
-    XFD_HIP(hipMemcpy(dst, src, cnt * sizeof(double2), hipMemcpyDeviceToHost));
+    readDoubles(*c, reinterpret_cast<const double*>(src), dst, static_cast<size_t>(2 * cnt));
   });
 }
 
@@ -3085,8 +3118,8 @@ int xfd_read_td_nf2ff(xfd_ctx* c, int32_t n, int32_t d, int32_t which, double* d
     require(c && dst && n >= 0 && n < static_cast<int32_t>(c->tdnfs.size()), "bad time-domain NF2FF index");
     require(d >= 0 && d < 6 && which >= 0 && which < 4, "bad time-domain NF2FF slice");
     auto& td = *c->tdnfs[n];
-    XFD_HIP(hipMemcpy(dst, td.pot.as<double>() + (static_cast<int64_t>(d) * 4 + which) * td.a.num,
-                      td.a.num * sizeof(double), hipMemcpyDeviceToHost));
+    readDoubles(*c, td.pot.as<double>() + (static_cast<int64_t>(d) * 4 + which) * td.a.num, dst,
+                static_cast<size_t>(td.a.num));
   });
 }
 

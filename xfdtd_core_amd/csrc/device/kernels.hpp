@@ -1032,16 +1032,19 @@ __global__ __launch_bounds__(256) void k_unpack(Grid g, const double* __restrict
   dst[g.at(u, v, w)] = static_cast<T>(src[t]);
 }
 
+// Elements [first, first + count) of a field's reference extent, to dst[0 ..
+// count) in the field's own precision: dst is pinned host memory, so the bytes
+// cross the bus once and the host widens them.
 template <class T>
-__global__ __launch_bounds__(256) void k_pack(Grid g, const T* __restrict__ src, double* dst, int n0, int n1,
-                                              int n2) {
-  const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int64_t vol = static_cast<int64_t>(n0) * n1 * n2;
-  if (t >= vol) return;
+__global__ __launch_bounds__(256) void k_pack(Grid g, const T* __restrict__ src, T* dst, int64_t first, int64_t count,
+                                              int n1, int n2) {
+  const int64_t q = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (q >= count) return;
+  const int64_t t = first + q;
   const int w = static_cast<int>(t % n2);
   const int v = static_cast<int>((t / n2) % n1);
   const int u = static_cast<int>(t / (static_cast<int64_t>(n2) * n1));
-  dst[t] = static_cast<double>(src[g.at(u, v, w)]);
+  dst[q] = src[g.at(u, v, w)];
 }
 
 // Time-domain NF2FF, phase 1, one thread per (group, cell):
@@ -1291,7 +1294,7 @@ struct Launch {
   static void far_field(hipStream_t s, const Nf2ffArgs& a, int f, const FarArgs& fa, int na, double* part,
                         double* out);
   static void unpack(hipStream_t s, const Grid& g, const double* src, T* dst, int n0, int n1, int n2);
-  static void pack(hipStream_t s, const Grid& g, const T* src, double* dst, int n0, int n1, int n2);
+  static void pack(hipStream_t s, const Grid& g, const T* src, T* dst, int64_t first, int64_t count, int n1, int n2);
 };
 
 }  // namespace xfd

@@ -246,10 +246,10 @@ void Launch<T>::unpack(hipStream_t s, const Grid& g, const double* src, T* dst, 
 }
 
 template <class T>
-void Launch<T>::pack(hipStream_t s, const Grid& g, const T* src, double* dst, int n0, int n1, int n2) {
-  const int64_t vol = static_cast<int64_t>(n0) * n1 * n2;
-  if (vol <= 0) return;
-  hipLaunchKernelGGL(k_pack<T>, dim3(blocks_for(vol, 256)), dim3(256), 0, s, g, src, dst, n0, n1, n2);
+void Launch<T>::pack(hipStream_t s, const Grid& g, const T* src, T* dst, int64_t first, int64_t count, int n1,
+                     int n2) {
+  if (count <= 0) return;
+  hipLaunchKernelGGL(k_pack<T>, dim3(blocks_for(count, 256)), dim3(256), 0, s, g, src, dst, first, count, n1, n2);
 }
 
 // ------------------------------------------------------------- batched --
