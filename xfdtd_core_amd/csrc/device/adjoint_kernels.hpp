@@ -400,8 +400,12 @@ __device__ __forceinline__ void adjMuCell(const Grid& g, const FieldPtrs<T>& L, 
   const int c = s.axis, a = (c + 1) % 3, b = (c + 2) % 3;
   const T cb = s.cb[p[c] - s.start];
   const int64_t idx = (static_cast<int64_t>(p[0]) * g.NY + p[1]) * g.pz + p[2];
-  if (p[a] < s.extA[0] && p[b] < s.extA[1]) s.psiA[t] = cb * s.psiA[t] + s.cpsiA[t] * L.f[s.fieldA][idx];
-  if (p[a] < s.extB[0] && p[b] < s.extB[1]) s.psiB[t] = cb * s.psiB[t] + s.cpsiB[t] * L.f[s.fieldB][idx];
+  using Pair = T __attribute__((ext_vector_type(2)));
+  Pair mu = reinterpret_cast<const Pair*>(s.psiA)[t];
+  const Pair c_psi = reinterpret_cast<const Pair*>(s.cpsiA)[t];
+  if (p[a] < s.extA[0] && p[b] < s.extA[1]) mu.x = cb * mu.x + c_psi.x * L.f[s.fieldA][idx];
+  if (p[a] < s.extB[0] && p[b] < s.extB[1]) mu.y = cb * mu.y + c_psi.y * L.f[s.fieldB][idx];
+  reinterpret_cast<Pair*>(s.psiA)[t] = mu;
 }
 
 // CPML adjoint, second half: the transpose of the psi difference.  E slab:
@@ -432,7 +436,7 @@ __device__ __forceinline__ void adjGatherCell(const Grid& g, const FieldPtrs<T>&
     if (pc < s.lo[c] || pc >= s.lo[c] + s.ext[c]) return -1;
     int q[3] = {p[0] - s.lo[0], p[1] - s.lo[1], p[2] - s.lo[2]};
     q[c] = pc - s.lo[c];
-    return (static_cast<int64_t>(q[0]) * s.ext[1] + q[1]) * s.ext[2] + q[2];
+    return 2 * ((static_cast<int64_t>(q[0]) * s.ext[1] + q[1]) * s.ext[2] + q[2]);
   };
   const int64_t tp = local(pin), tm = local(pout);
   // component A of the slab reads dual B; component B reads dual A

@@ -248,8 +248,10 @@ struct xfd_ctx {
     int axis, n, e_start, h_start;
     int lo_e[3], lo_h[3], ext[3] = {0, 0, 0}, ext_h[3] = {0, 0, 0};
     int extA_e[2], extB_e[2], extA_h[2], extB_h[2];
-    DevBuf cpsi[4], psi[4];  // ea_hb, eb_ha, ha_eb, hb_ea (box layout)
-    DevBuf psi_h2[2];        // the single-pass step's second set of ha_eb, hb_ea
+    // E (ea_hb, eb_ha) and H (ha_eb, hb_ea), the two components' values of a
+    // point side by side: one access each for psi and c_psi, half the lines
+    DevBuf cpsi[2], psi[2];
+    DevBuf psi_h2;  // the single-pass step's second set of the H psi
     DevBuf ae, be, ah, bh;
   };
   std::vector<std::unique_ptr<Slab>> slabs;
@@ -462,16 +464,13 @@ void leaveStep(xfd_ctx& c) {
     for (int f = 0; f < 6; ++f)
       XFD_HIP(hipMemcpyAsync(c.fields[f].p, c.fields_b[f].p, c.fields[f].bytes, hipMemcpyDeviceToDevice, c.stream));
     for (auto& sl : c.slabs)
-      for (int q = 0; q < 2; ++q)
-        XFD_HIP(hipMemcpyAsync(sl->psi[2 + q].p, sl->psi_h2[q].p, sl->psi[2 + q].bytes, hipMemcpyDeviceToDevice,
-                               c.stream));
+      XFD_HIP(hipMemcpyAsync(sl->psi[1].p, sl->psi_h2.p, sl->psi[1].bytes, hipMemcpyDeviceToDevice, c.stream));
     XFD_HIP(hipStreamSynchronize(c.stream));
   }
   c.parity = 0;
   c.fstep = false;
   for (auto& f : c.fields_b) f.reset();
-  for (auto& sl : c.slabs)
-    for (auto& b : sl->psi_h2) b.reset();
+  for (auto& sl : c.slabs) sl->psi_h2.reset();
 }
 
 // The dispersive update's arguments (zero when the context has no ADE).
@@ -737,6 +736,17 @@ void listByBin(int64_t bins, size_t count, F&& bin, DevBuf& off, DevBuf& of) {
   uploadVector(list, of);
 }
 
+// The tile of tk x tj x ti points (k, j, i) that a padded index lies in; a point
+// on a far plane (a probe's) goes to the nearest tile.
+int64_t tileOf(const xfd::Grid& g, int64_t x, int64_t tk, int64_t tj, int64_t ti) {
+  int64_t p[3];
+  g.point(x, p);
+  const int64_t i = std::min<int64_t>(p[0], g.nx - 1), j = std::min<int64_t>(p[1], g.ny - 1),
+                k = std::min<int64_t>(p[2], g.nz - 1);
+  const int64_t nbx = (g.nz + tk - 1) / tk, nby = (g.ny + tj - 1) / tj;
+  return (i / ti * nby + j / tj) * nbx + k / tk;
+}
+
 // Chooses the 1D kernel that steps many times in one launch (k_line): every
 // correction on Ex or Hy of the column (0, 0), or of (0, 1) away from the CPML
 // layers (a TFSF face corrects both), every probe one of those two,
@@ -850,13 +860,9 @@ void halfSetup(xfd_ctx& c, const std::vector<xfd::Record>& re, const std::vector
     tiles = nbx * ((g.nx + rows - 1) / rows);
   }
   require(tiles < (int64_t{1} << 31), "grid too large");
-  auto tile = [&](int64_t x) {  // a probe on a far plane goes to the nearest tile
-    int64_t p[3];
-    g.point(x, p);
-    const int64_t i = std::min<int64_t>(p[0], g.nx - 1), j = std::min<int64_t>(p[1], g.ny - 1),
-                  k = std::min<int64_t>(p[2], g.nz - 1);
-    if (c.dim == 2) return i / (xfd::kTeRows * c.half_chunk) * nbx + j / 64;
-    return (i / c.half_chunk * nby + j / c.half_tj) * nbx + k / c.half_tk;
+  auto tile = [&](int64_t x) {
+    return c.dim == 2 ? tileOf(g, x, 1, 64, xfd::kTeRows * c.half_chunk)
+                      : tileOf(g, x, c.half_tk, c.half_tj, c.half_chunk);
   };
   listByBin(tiles, static_cast<size_t>(c.nseg_e), [&](size_t q) { return tile(re[se[q]].target); }, c.rec_off_e, c.seg_of_e);
   listByBin(tiles, static_cast<size_t>(c.nseg_h), [&](size_t q) { return tile(rh[sh[q]].target); }, c.rec_off_h, c.seg_of_h);
@@ -969,25 +975,27 @@ void createTyped(xfd_ctx& c, const xfd_desc& d) {
     const double* src[4] = {p.c_ea_psi_hb, p.c_eb_psi_ha, p.c_ha_psi_eb, p.c_hb_psi_ea};
     // psi extents in (a, b) per array
     const int pe[4][2] = {{N[a], N[b] + 1}, {N[a] + 1, N[b]}, {N[a] + 1, N[b]}, {N[a], N[b] + 1}};
-    for (int q = 0; q < 4; ++q) {
-      require(src[q] != nullptr, "CPML c_psi array missing");
-      std::vector<T> box(vol, T(0));
-      // reference psi arrays are xyz-ordered with the layer index on the
-      // main axis (pml.cpp:297-337)
-      int ex[3];
-      ex[cax] = p.n;
-      ex[a] = pe[q][0];
-      ex[b] = pe[q][1];
-      for (int64_t x = 0; x < ex[0]; ++x)
-        for (int64_t y = 0; y < ex[1]; ++y)
-          for (int64_t z = 0; z < ex[2]; ++z) {
-            const int64_t lin = (x * ex[1] + y) * ex[2] + z;
-            // box-local: the main axis starts at the slab start in both boxes
-            const int64_t t = (x * s->ext[1] + y) * s->ext[2] + z;
-            box[t] = static_cast<T>(src[q][lin]);
-          }
-      uploadVector(box, s->cpsi[q]);
-      s->psi[q].alloc(vol * sizeof(T));
+    for (int half = 0; half < 2; ++half) {
+      std::vector<T> box(2 * vol, T(0));
+      for (int q = 2 * half; q < 2 * half + 2; ++q) {
+        require(src[q] != nullptr, "CPML c_psi array missing");
+        // reference psi arrays are xyz-ordered with the layer index on the
+        // main axis (pml.cpp:297-337)
+        int ex[3];
+        ex[cax] = p.n;
+        ex[a] = pe[q][0];
+        ex[b] = pe[q][1];
+        for (int64_t x = 0; x < ex[0]; ++x)
+          for (int64_t y = 0; y < ex[1]; ++y)
+            for (int64_t z = 0; z < ex[2]; ++z) {
+              const int64_t lin = (x * ex[1] + y) * ex[2] + z;
+              // box-local: the main axis starts at the slab start in both boxes
+              const int64_t t = (x * s->ext[1] + y) * s->ext[2] + z;
+              box[2 * t + q % 2] = static_cast<T>(src[q][lin]);
+            }
+      }
+      uploadVector(box, s->cpsi[half]);
+      s->psi[half].alloc(2 * vol * sizeof(T));
     }
     auto up = [&](const double* v, DevBuf& b) {
       require(v != nullptr, "CPML profile missing");
@@ -1457,8 +1465,7 @@ void createTyped(xfd_ctx& c, const xfd_desc& d) {
         c.fstep_chunk = v;
       }
       for (int f = 0; f < 6; ++f) c.fields_b[f].alloc(c.fields[f].bytes);
-      for (auto& sl : c.slabs)
-        for (int q = 0; q < 2; ++q) sl->psi_h2[q].alloc(sl->psi[2 + q].bytes);
+      for (auto& sl : c.slabs) sl->psi_h2.alloc(sl->psi[1].bytes);
       c.parity = 0;
     }
   }
@@ -1497,8 +1504,8 @@ xfd::StepSlabs<T> stepSlabs(xfd_ctx& c, bool is_e) {
       S.rdA = S.wrA = a.psiA;
       S.rdB = S.wrB = a.psiB;
     } else {
-      T* cur[2] = {sp->psi[2].as<T>(), sp->psi[3].as<T>()};
-      T* alt[2] = {sp->psi_h2[0].as<T>(), sp->psi_h2[1].as<T>()};
+      T* cur[2] = {sp->psi[1].as<T>(), sp->psi[1].as<T>() + 1};
+      T* alt[2] = {sp->psi_h2.as<T>(), sp->psi_h2.as<T>() + 1};
       S.rdA = c.parity ? alt[0] : cur[0];
       S.rdB = c.parity ? alt[1] : cur[1];
       S.wrA = c.parity ? cur[0] : alt[0];
@@ -1529,9 +1536,7 @@ xfd::SlabArgs<T> slabArgs(xfd_ctx::Slab& s, bool is_e) {
     a.dualA = 3 + ta;
     a.dualB = 3 + tb;
     a.cpsiA = s.cpsi[0].as<T>();
-    a.cpsiB = s.cpsi[1].as<T>();
     a.psiA = s.psi[0].as<T>();
-    a.psiB = s.psi[1].as<T>();
     a.ca = s.ae.as<T>();
     a.cb = s.be.as<T>();
   } else {
@@ -1543,13 +1548,13 @@ xfd::SlabArgs<T> slabArgs(xfd_ctx::Slab& s, bool is_e) {
     a.fieldB = 3 + tb;
     a.dualA = ta;
     a.dualB = tb;
-    a.cpsiA = s.cpsi[2].as<T>();
-    a.cpsiB = s.cpsi[3].as<T>();
-    a.psiA = s.psi[2].as<T>();
-    a.psiB = s.psi[3].as<T>();
+    a.cpsiA = s.cpsi[1].as<T>();
+    a.psiA = s.psi[1].as<T>();
     a.ca = s.ah.as<T>();
     a.cb = s.bh.as<T>();
   }
+  a.cpsiB = a.cpsiA + 1;
+  a.psiB = a.psiA + 1;
   return a;
 }
 
@@ -1564,7 +1569,7 @@ xfd::ZSlab<T> zSlab(const xfd::SlabArgs<T>& a, const xfd::Grid& g) {
               a.extA[0] >= g.nx && a.extA[1] >= g.ny && a.extB[0] >= g.nx && a.extB[1] >= g.ny &&
               a.lo[2] == a.start && a.ext[2] == a.n,
           "z CPML slab shape");
-  require(static_cast<int64_t>(a.ext[0]) * a.ext[1] * a.ext[2] < (int64_t{1} << 31), "z CPML slab too large");
+  require(static_cast<int64_t>(a.ext[0]) * a.ext[1] * a.ext[2] < (int64_t{1} << 30), "z CPML slab too large");
   xfd::ZSlab<T> z{};
   z.klo = a.start;
   z.khi = a.start + a.n;
@@ -1613,7 +1618,7 @@ std::vector<xfd::HalfSlabs<T>> halfSlabs(xfd_ctx& c, bool is_e) {
   for (int ax = 0; ax < 3; ++ax)
     for (int q = 0; q < H.n[ax]; ++q) {
       const auto s = slabArgs<T>(*c.slabs[slab[ax][q]], is_e);
-      H.s[ax][q] = {s.start, s.start + s.n, s.ca, s.cb, s.cpsiA, s.cpsiB, s.psiA, s.psiB};
+      H.s[ax][q] = {s.start, s.start + s.n, s.ca, s.cb, s.cpsiA, s.psiA};
     }
   return v;
 }
@@ -1941,7 +1946,7 @@ void resetState(xfd_ctx& c) {
   for (auto& f : c.fields_b) zero(f);
   for (auto& sl : c.slabs) {
     for (auto& p : sl->psi) zero(p);
-    for (auto& p : sl->psi_h2) zero(p);
+    zero(sl->psi_h2);
   }
   c.parity = 0;
   zero(c.state);
@@ -2092,15 +2097,15 @@ void backwardTyped(xfd_ctx& c, const xfd_adjoint_desc& D, double* grad_out) {
   std::vector<xfd::SlabArgs<T>> me, mh;
   const int64_t stride[3] = {c.g.plane, c.g.pz, 1};
   for (auto& sl : c.slabs) {
-    mu.emplace_back(new DevBuf[4]);
-    for (int q = 0; q < 4; ++q) mu.back()[q].alloc(sl->psi[q].bytes);
+    mu.emplace_back(new DevBuf[2]);
+    for (int q = 0; q < 2; ++q) mu.back()[q].alloc(sl->psi[q].bytes);
     auto e = slabArgs<T>(*sl, true), h = slabArgs<T>(*sl, false);
     e.stride_c = stride[e.axis];
     h.stride_c = stride[h.axis];
     e.psiA = mu.back()[0].as<T>();
-    e.psiB = mu.back()[1].as<T>();
-    h.psiA = mu.back()[2].as<T>();
-    h.psiB = mu.back()[3].as<T>();
+    e.psiB = e.psiA + 1;
+    h.psiA = mu.back()[1].as<T>();
+    h.psiB = h.psiA + 1;
     me.push_back(e);
     mh.push_back(h);
   }
@@ -2999,10 +3004,12 @@ int xfd_batch_create(int32_t n, const xfd_desc* descs, xfd_batch** out) {
       if (xfd_create(&descs[i], &c) != XFD_OK) throw XfdError(XFD_EINVAL, std::string("case ") + std::to_string(i) + ": " + g_err);
       b->cases.emplace_back(c);
       leaveStep(*c);  // the batched launches step set 0 with their own tables
+      // Batched cases keep their slabs and records as separate launches: with
+      // half of these small boxes' points in a slab, all cases' half-steps in
+      // one launch took 203 us where sweep, slabs and records take 210 (16 cases
+      // of 48..128 cells a side, FP32), and the sweeps with only the z slabs
+      // inside were slower.
       c->half = false;
-      // batched cases keep their z slabs as separate launches: with most
-      // wavefronts of these small boxes carrying slab lanes, the sweeps were
-      // measured slower with them inside
       c->zfused = false;
       std::fill(c->zslab.begin(), c->zslab.end(), 0);
       b->shared = b->shared && c->classed && !c->wide && c->tdnfs.empty();

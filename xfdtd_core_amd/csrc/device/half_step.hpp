@@ -20,29 +20,36 @@
 // The far planes i = nx, j = ny, k = nz are left out: their slab corrections
 // draw on each other only, so the zeros they start with stay.
 //
-// Measured, us per step of both half-steps with separate launches / this (wall
-// time): 63^3 FP64 with a TFSF box 55 / 30, 100^3 FP32 66 / 38, 128^3 FP64 117 /
-// 82, 384^3 FP32 1082 / 1025.  Loading plane i + 1 during plane i was tried: no
+// psi and c_psi hold both components of a point side by side: one access each
+// where there were two, and half the lines of a z slab's short rows.
+//
+// Measured, us per step (kernel time), separate launches / this: 63^3 FP64 with
+// a TFSF box 55 / 24, 100^3 FP32 66 / 35, 128^3 FP64 117 / 92, 203 x 181 x 225
+// FP64 410 / 385, 384^3 FP32 1082 / 1041 (a half-step without its slabs: 435, so
+// they cost 85 for 256 MB).  With the components apart: 100^3 37.1, 128^3 99.5,
+// 203 x 181 x 225 407.  Rows padded to whole lines instead were slower (216 at
+// 203 x 181 x 225, FP64), as were registers capped for one more wavefront per
+// SIMD (spills: 384^3 690 a half-step).  Loading plane i + 1 during plane i was tried: no
 // faster on small boxes and 2 % slower at 384^3 (fewer wavefronts per CU).
 #pragma once
+
+#include <climits>
 
 #include "kernels.hpp"
 
 namespace xfd {
 
 // One CPML slab: layers [lo, hi) along its axis, the recursive-convolution
-// coefficients per layer, and c_psi / psi of its components A = (axis+1)%3
-// and B = (axis+2)%3 in the slab's box layout (k fastest; the box spans N + 1
-// points along the other two axes).
+// coefficients per layer, and c_psi / psi of its components A = (axis+1)%3 and
+// B = (axis+2)%3, a pair per point, in the slab's box layout (k fastest; the box
+// spans N + 1 points along the other two axes).
 template <class T>
 struct AxisSlab {
   int lo, hi;
   const T* ca;
   const T* cb;
-  const T* cA;
-  const T* cB;
-  T* pA;
-  T* pB;
+  const T* c;
+  T* psi;
 };
 
 // The slabs of one half-step, per axis in position order.  Component q is
@@ -79,9 +86,18 @@ struct SlabVals {
   T pA = T(0), pB = T(0), cA = T(0), cB = T(0);
 };
 
+// Both components of a point in one access.
 template <class T>
-__device__ __forceinline__ SlabVals<T> slabLoad(const AxisSlab<T>& s, int64_t u, unsigned e) {
-  return SlabVals<T>{(s.pA + u)[e], (s.pB + u)[e], (s.cA + u)[e], (s.cB + u)[e]};
+struct alignas(2 * sizeof(T)) SlabPair {
+  T a, b;
+};
+
+// u: uniform point offset in the box, e: the lane's
+template <class T>
+__device__ __forceinline__ SlabVals<T> slabLoad(const T* c, const T* psi, int64_t u, unsigned e) {
+  const SlabPair<T> p = (reinterpret_cast<const SlabPair<T>*>(psi) + u)[e];
+  const SlabPair<T> q = (reinterpret_cast<const SlabPair<T>*>(c) + u)[e];
+  return SlabVals<T>{p.a, p.b, q.a, q.b};
 }
 
 // a b + c: fused in FP32, two roundings in FP64 (the reference's).  Explicit,
@@ -95,13 +111,11 @@ __device__ __forceinline__ double mulAdd(double a, double b, double c) {
 
 // psi = b psi + a d for both components of a slab point, stored.
 template <class T>
-__device__ __forceinline__ void slabStore(const AxisSlab<T>& s, int64_t u, unsigned e, SlabVals<T>& v, T ca, T cb,
-                                          T dA, T dB) {
+__device__ __forceinline__ void slabStore(T* psi, int64_t u, unsigned e, SlabVals<T>& v, T ca, T cb, T dA, T dB) {
 #pragma clang fp contract(off)
   v.pA = mulAdd(ca, dA, cb * v.pA);
   v.pB = mulAdd(ca, dB, cb * v.pB);
-  (s.pA + u)[e] = v.pA;
-  (s.pB + u)[e] = v.pB;
+  (reinterpret_cast<SlabPair<T>*>(psi) + u)[e] = SlabPair<T>{v.pA, v.pB};
 }
 
 // v + ca pa + cb pb, the latter first where the boundary's order swaps them.
@@ -125,9 +139,12 @@ struct HalfPlane {
 };
 
 // One tile of a half-step: TK lanes along k, TJ rows along j, planes
-// [i0, i0 + ichunk).  S: the dispersive scheme of the E half-step, or -1.
-template <class T, class Coef, bool IsE, int S, bool NT, int TK, int TJ>
-__device__ __forceinline__ void halfTile(const Grid& g, const FieldPtrs<T>& F, const Coef& C, const AdeArgs<T>& A,
+// [i0, i0 + ichunk).  S: the dispersive scheme of the E half-step, or -1; P: the
+// most poles whose currents a dispersive cell loads at once (its registers
+// bound the wavefronts in flight: 160^3 FP32 with two poles, 133 us against 150 us
+// with room for four).
+template <class T, class Coef, bool IsE, int S, bool NT, int TK, int TJ, int P = kAdeFastPoles>
+__device__ __forceinline__ void halfTile(const Grid g, const FieldPtrs<T> F, const Coef C, const AdeArgs<T> A,
                                          const HalfSlabs<T>* __restrict__ HP, int bx, int by, int bz, int ichunk) {
 #pragma clang fp contract(off)
   static_assert(TK % 64 == 0, "a wavefront is part of one row");
@@ -141,9 +158,19 @@ __device__ __forceinline__ void halfTile(const Grid& g, const FieldPtrs<T>& F, c
   int64_t u = (static_cast<int64_t>(i0) * g.NY + j) * pz + k0;  // uniform; the lane's element is u + lane
   // slabs: the x slab of the march (re-picked where the march leaves it), the
   // row's y slab and the lane's z slab
-  int xq = H.n[0] > 1 && i0 >= H.s[0][0].hi ? 1 : 0;
-  const bool inY0 = H.n[1] > 0 && j >= H.s[1][0].lo && j < H.s[1][0].hi;
-  const bool inY1 = H.n[1] > 1 && j >= H.s[1][1].lo && j < H.s[1][1].hi;
+  // The bounds that every plane tests are copies: memory that the stores below
+  // might alias would be read again, a chain of scalar loads, in every plane.
+  // The slabs' pointers stay in memory: as copies they cost registers (384^3
+  // FP32 525 against 520 us a half-step).
+  const int nx = H.n[0], ny = H.n[1], nz = H.n[2];
+  const int swap0 = H.swap[0], swap1 = H.swap[1], swap2 = H.swap[2];
+  const int xend = nx > 1 ? H.s[0][0].hi : INT_MAX;  // where the march passes to the far x slab
+  bool second = i0 >= xend;
+  const AxisSlab<T>* xs = &H.s[0][second ? 1 : 0];
+  int xlo = nx > 0 ? xs->lo : INT_MAX, xhi = nx > 0 ? xs->hi : 0;
+  const AxisSlab<T>&Z0 = H.s[2][0], &Z1 = H.s[2][1];
+  const bool inY0 = ny > 0 && j >= H.s[1][0].lo && j < H.s[1][0].hi;
+  const bool inY1 = ny > 1 && j >= H.s[1][1].lo && j < H.s[1][1].hi;
   const bool inY = inY0 || inY1;
   const AxisSlab<T>& Y = H.s[1][inY1 ? 1 : 0];
   T yca = T(0), ycb = T(0);
@@ -154,30 +181,28 @@ __device__ __forceinline__ void halfTile(const Grid& g, const FieldPtrs<T>& F, c
     yp = static_cast<int64_t>(Y.hi - Y.lo) * (g.nz + 1);
     yu = i0 * yp + static_cast<int64_t>(j - Y.lo) * (g.nz + 1) + k0;
   }
-  const bool inZ0 = H.n[2] > 0 && k >= H.s[2][0].lo && k < H.s[2][0].hi;
-  const bool inZ1 = H.n[2] > 1 && k >= H.s[2][1].lo && k < H.s[2][1].hi;
+  const bool inZ0 = nz > 0 && k >= Z0.lo && k < Z0.hi;
+  const bool inZ1 = nz > 1 && k >= Z1.lo && k < Z1.hi;
   T zca = T(0), zcb = T(0);
   unsigned ze = 0;
   int64_t zu0 = 0, zu1 = 0, zp0 = 0, zp1 = 0;
   if (inZ0) {
-    const AxisSlab<T>& Z = H.s[2][0];
-    ze = static_cast<unsigned>(k - Z.lo);
-    zca = Z.ca[ze];
-    zcb = Z.cb[ze];
+    ze = static_cast<unsigned>(k - Z0.lo);
+    zca = Z0.ca[ze];
+    zcb = Z0.cb[ze];
   }
   if (inZ1) {
-    const AxisSlab<T>& Z = H.s[2][1];
-    ze = static_cast<unsigned>(k - Z.lo);
-    zca = Z.ca[ze];
-    zcb = Z.cb[ze];
+    ze = static_cast<unsigned>(k - Z1.lo);
+    zca = Z1.ca[ze];
+    zcb = Z1.cb[ze];
   }
-  if (H.n[2] > 0) {
-    const int n0 = H.s[2][0].hi - H.s[2][0].lo;
+  if (nz > 0) {
+    const int n0 = Z0.hi - Z0.lo;
     zp0 = static_cast<int64_t>(g.NY) * n0;
     zu0 = i0 * zp0 + static_cast<int64_t>(j) * n0;
   }
-  if (H.n[2] > 1) {
-    const int n1 = H.s[2][1].hi - H.s[2][1].lo;
+  if (nz > 1) {
+    const int n1 = Z1.hi - Z1.lo;
     zp1 = static_cast<int64_t>(g.NY) * n1;
     zu1 = i0 * zp1 + static_cast<int64_t>(j) * n1;
   }
@@ -205,10 +230,10 @@ __device__ __forceinline__ void halfTile(const Grid& g, const FieldPtrs<T>& F, c
   const unsigned ek = lane + (IsE && k == 0 ? 1u : 0u);
   auto load = [&](int64_t w) {
     HalfPlane<T, Coef> p;
-    p.r0 = C.template raw<NT>(q0, w + lane);
-    p.r1 = C.template raw<NT>(q0 + 1, w + lane);
-    p.r2 = C.template raw<NT>(q0 + 2, w + lane);
-    p.m = S >= 0 ? ldOwn<NT>(A.mat + w + lane) : -1;
+    p.r0 = C.template rawAt<NT>(q0, w, lane);
+    p.r1 = C.template rawAt<NT>(q0 + 1, w, lane);
+    p.r2 = C.template rawAt<NT>(q0 + 2, w, lane);
+    p.m = S >= 0 ? ldOwn<NT>((A.mat + w) + lane) : -1;
     p.a0 = (d0 + w)[lane];
     p.b1 = (d1 + (IsE ? w : w + pl))[lane];
     p.b2 = (d2 + (IsE ? w : w + pl))[lane];
@@ -216,20 +241,25 @@ __device__ __forceinline__ void halfTile(const Grid& g, const FieldPtrs<T>& F, c
     p.j2 = (d2 + (w + dj))[lane];
     p.k0 = (d0 + (w + uk))[ek];
     p.k1 = (d1 + (w + uk))[ek];
-    p.o0 = ldOwn<NT>(f0 + w + lane);
-    p.o1 = ldOwn<NT>(f1 + w + lane);
-    p.o2 = ldOwn<NT>(f2 + w + lane);
+    p.o0 = ldOwn<NT>((f0 + w) + lane);
+    p.o1 = ldOwn<NT>((f1 + w) + lane);
+    p.o2 = ldOwn<NT>((f2 + w) + lane);
     return p;
   };
   for (int i = i0; i < i1; ++i, u += pl) {
-    const HalfPlane<T, Coef> P = load(u);  // every load of the plane first
+    const HalfPlane<T, Coef> L = load(u);  // every load of the plane first
     T s0, p0, r0, s1, p1, r1, s2, p2, r2;
-    C.resolve(q0, P.r0, s0, p0, r0);
-    C.resolve(q0 + 1, P.r1, s1, p1, r1);
-    C.resolve(q0 + 2, P.r2, s2, p2, r2);
-    if (xq == 0 && H.n[0] > 1 && i >= H.s[0][0].hi) xq = 1;
-    const AxisSlab<T>& X = H.s[0][xq];
-    const bool inX = H.n[0] > 0 && i >= X.lo && i < X.hi;
+    C.resolveAt(q0, L.r0, s0, p0, r0);
+    C.resolveAt(q0 + 1, L.r1, s1, p1, r1);
+    C.resolveAt(q0 + 2, L.r2, s2, p2, r2);
+    if (i >= xend && !second) {
+      second = true;
+      xs = &H.s[0][1];
+      xlo = xs->lo;
+      xhi = xs->hi;
+    }
+    const AxisSlab<T>& X = *xs;
+    const bool inX = i >= xlo && i < xhi;
     SlabVals<T> sx, sy, sz;
     T xca = T(0), xcb = T(0);
     int64_t xu = 0;
@@ -237,18 +267,18 @@ __device__ __forceinline__ void halfTile(const Grid& g, const FieldPtrs<T>& F, c
       xca = X.ca[i - X.lo];
       xcb = X.cb[i - X.lo];
       xu = (static_cast<int64_t>(i - X.lo) * g.NY + j) * (g.nz + 1) + k0;
-      sx = slabLoad(X, xu, lane);
+      sx = slabLoad<T>(X.c, X.psi, xu, lane);
     }
-    if (inY) sy = slabLoad(Y, yu, lane);
-    if (inZ0) sz = slabLoad(H.s[2][0], zu0, ze);
-    if (inZ1) sz = slabLoad(H.s[2][1], zu1, ze);
-    const int m = P.m;
-    const T a0 = P.a0, o0 = P.o0, o1 = P.o1, o2 = P.o2;
+    if (inY) sy = slabLoad<T>(Y.c, Y.psi, yu, lane);
+    if (inZ0) sz = slabLoad<T>(Z0.c, Z0.psi, zu0, ze);
+    if (inZ1) sz = slabLoad<T>(Z1.c, Z1.psi, zu1, ze);
+    const int m = L.m;
+    const T a0 = L.a0, o0 = L.o0, o1 = L.o1, o2 = L.o2;
     // differences of dual component q along axis x, y, z
-    const T x1 = P.b1 - c1, x2 = P.b2 - c2;
-    const T b1 = IsE ? P.b1 : c1, b2 = IsE ? P.b2 : c2;
-    const T y0 = IsE ? a0 - P.j0 : P.j0 - a0, y2 = IsE ? b2 - P.j2 : P.j2 - b2;
-    const T z0 = IsE ? a0 - P.k0 : P.k0 - a0, z1 = IsE ? b1 - P.k1 : P.k1 - b1;
+    const T x1 = L.b1 - c1, x2 = L.b2 - c2;
+    const T b1 = IsE ? L.b1 : c1, b2 = IsE ? L.b2 : c2;
+    const T y0 = IsE ? a0 - L.j0 : L.j0 - a0, y2 = IsE ? b2 - L.j2 : L.j2 - b2;
+    const T z0 = IsE ? a0 - L.k0 : L.k0 - a0, z1 = IsE ? b1 - L.k1 : L.k1 - b1;
     // component 0: d1 along z, d2 along y; 1: d2 along x, d0 along z; 2: d0 along y, d1 along x
     const T w0 = mulAdd(r0, y2, mulAdd(p0, z1, s0 * o0));
     const T w1 = mulAdd(r1, z0, mulAdd(p1, x2, s1 * o1));
@@ -263,8 +293,8 @@ __device__ __forceinline__ void halfTile(const Grid& g, const FieldPtrs<T>& F, c
       } else {
         const T cur[3] = {o0, o1, o2}, en[3] = {w0, w1, w2};
         T v[3];
-        if (A.poles <= kAdeFastPoles) {
-          adeCell<T, S < 0 ? 0 : S>(A, m, u + lane, r, cur, en, v);
+        if (A.poles <= P) {
+          adeCell<T, S < 0 ? 0 : S, P>(A, m, u + lane, r, cur, en, v);
         } else {
 #pragma unroll
           for (int q = 0; q < 3; ++q) v[q] = r[q] ? adeUpdate<T, S < 0 ? 0 : S>(A, m, q, u + lane, cur[q], en[q]) : cur[q];
@@ -276,18 +306,18 @@ __device__ __forceinline__ void halfTile(const Grid& g, const FieldPtrs<T>& F, c
     }
     // x: components 1 (dual 2) and 2 (dual 1); y: 2 (dual 0) and 0 (dual 2);
     // z: 0 (dual 1) and 1 (dual 0)
-    if (inX) slabStore(X, xu, lane, sx, xca, xcb, x2, x1);
-    if (inY) slabStore(Y, yu, lane, sy, yca, ycb, y0, y2);
-    if (inZ0) slabStore(H.s[2][0], zu0, ze, sz, zca, zcb, z1, z0);
-    if (inZ1) slabStore(H.s[2][1], zu1, ze, sz, zca, zcb, z1, z0);
-    v0 = addInOrder(v0, sy.cB, sy.pB, sz.cA, sz.pA, H.swap[0]);
-    v1 = addInOrder(v1, sz.cB, sz.pB, sx.cA, sx.pA, H.swap[1]);
-    v2 = addInOrder(v2, sx.cB, sx.pB, sy.cA, sy.pA, H.swap[2]);
-    stOwn<NT>(f0 + u + lane, v0);
-    stOwn<NT>(f1 + u + lane, v1);
-    stOwn<NT>(f2 + u + lane, v2);
-    c1 = P.b1;
-    c2 = P.b2;
+    if (inX) slabStore(X.psi, xu, lane, sx, xca, xcb, x2, x1);
+    if (inY) slabStore(Y.psi, yu, lane, sy, yca, ycb, y0, y2);
+    if (inZ0) slabStore(Z0.psi, zu0, ze, sz, zca, zcb, z1, z0);
+    if (inZ1) slabStore(Z1.psi, zu1, ze, sz, zca, zcb, z1, z0);
+    v0 = addInOrder(v0, sy.cB, sy.pB, sz.cA, sz.pA, swap0);
+    v1 = addInOrder(v1, sz.cB, sz.pB, sx.cA, sx.pA, swap1);
+    v2 = addInOrder(v2, sx.cB, sx.pB, sy.cA, sy.pA, swap2);
+    stOwn<NT>((f0 + u) + lane, v0);
+    stOwn<NT>((f1 + u) + lane, v1);
+    stOwn<NT>((f2 + u) + lane, v2);
+    c1 = L.b1;
+    c2 = L.b2;
     yu += yp;
     zu0 += zp0;
     zu1 += zp1;
@@ -322,12 +352,12 @@ __device__ __forceinline__ void halfEvents(const FieldPtrs<T>& F, const HalfEven
   }
 }
 
-template <class T, class Coef, bool IsE, int S, bool NT, int TK, int TJ>
+template <class T, class Coef, bool IsE, int S, bool NT, int TK, int TJ, int P = kAdeFastPoles>
 __global__ __launch_bounds__(TK * TJ) void k_half(Grid g, FieldPtrs<T> F, Coef C, AdeArgs<T> A, const HalfSlabs<T>* H,
                                                   HalfEvents<T> ev, SweepMap M, int ichunk, int64_t t) {
   int bx, by, bz;
   M.coords(bx, by, bz);
-  halfTile<T, Coef, IsE, S, NT, TK, TJ>(g, F, C, A, H, bx, by, bz, ichunk);
+  halfTile<T, Coef, IsE, S, NT, TK, TJ, P>(g, F, C, A, H, bx, by, bz, ichunk);
   halfEvents(F, ev, (static_cast<int64_t>(bz) * M.nby + by) * M.nbx + bx, t);
 }
 

@@ -77,7 +77,7 @@ __device__ __forceinline__ void cpmlFused(const CpmlList<T>& P, uint32_t mask, i
     const int u = i - S.lo[0];
     if (u < 0 || u >= S.ext[0]) continue;
     const int c = S.axis, a = c == 2 ? 0 : c + 1, b = c == 0 ? 2 : c - 1;
-    const int64_t t = (static_cast<int64_t>(u) * S.ext[1] + (j - S.lo[1])) * S.ext[2] + (k - S.lo[2]);
+    const int64_t t = 2 * ((static_cast<int64_t>(u) * S.ext[1] + (j - S.lo[1])) * S.ext[2] + (k - S.lo[2]));
     const int layer = pick3(c, i, j, k) - S.start;
     const int pa = pick3(a, i, j, k), pb = pick3(b, i, j, k);
     const T ca = S.ca[layer], cb = S.cb[layer];
@@ -134,8 +134,8 @@ __device__ __forceinline__ ZLane<T> zLane(const ZCpml<T>& Z, int i0, int j, int 
   const T* cb = in1 ? s1.cb : s0.cb;
   L.ca = ca[k - klo];
   L.cb = cb[k - klo];
-  L.step = ext1 * ext2;
-  L.t = (i0 * ext1 + j) * ext2 + (k - klo);
+  L.step = 2 * ext1 * ext2;
+  L.t = 2 * ((i0 * ext1 + j) * ext2 + (k - klo));
   return L;
 }
 
@@ -492,22 +492,22 @@ __device__ __forceinline__ void cpmlPoint(const Grid& g, const FieldPtrs<T>& F, 
   const int64_t idx = g.at(p0, p1, p2);
   const int64_t q = IsE ? idx - s.stride_c : idx + s.stride_c;
   const int pa = pick3(a, p0, p1, p2), pb = pick3(b, p0, p1, p2);
-  if (pa < s.extA[0] && pb < s.extA[1]) {
+  const bool inA = pa < s.extA[0] && pb < s.extA[1], inB = pa < s.extB[0] && pb < s.extB[1];
+  if (!inA && !inB) return;
+  using Pair = T __attribute__((ext_vector_type(2)));
+  Pair psi = ldOwn(reinterpret_cast<const Pair*>(s.psiA + t));
+  const Pair c_psi = ldOwn(reinterpret_cast<const Pair*>(s.cpsiA + t));
+  if (inA) {
     const T* dual = F.f[s.dualB];
-    T psi = ldOwn(s.psiA + t);
-    psi = IsE ? cb * psi + ca * (dual[idx] - dual[q]) : cb * psi + ca * (dual[q] - dual[idx]);
-    stOwn(s.psiA + t, psi);
-    T* f = F.f[s.fieldA];
-    f[idx] += ldOwn(s.cpsiA + t) * psi;
+    psi.x = IsE ? cb * psi.x + ca * (dual[idx] - dual[q]) : cb * psi.x + ca * (dual[q] - dual[idx]);
+    F.f[s.fieldA][idx] += c_psi.x * psi.x;
   }
-  if (pa < s.extB[0] && pb < s.extB[1]) {
+  if (inB) {
     const T* dual = F.f[s.dualA];
-    T psi = ldOwn(s.psiB + t);
-    psi = IsE ? cb * psi + ca * (dual[idx] - dual[q]) : cb * psi + ca * (dual[q] - dual[idx]);
-    stOwn(s.psiB + t, psi);
-    T* f = F.f[s.fieldB];
-    f[idx] += ldOwn(s.cpsiB + t) * psi;
+    psi.y = IsE ? cb * psi.y + ca * (dual[idx] - dual[q]) : cb * psi.y + ca * (dual[q] - dual[idx]);
+    F.f[s.fieldB][idx] += c_psi.y * psi.y;
   }
+  stOwn(reinterpret_cast<Pair*>(s.psiA + t), psi);
 }
 
 template <class T, bool IsE>
@@ -517,7 +517,7 @@ __device__ __forceinline__ void cpmlCell(const Grid& g, const FieldPtrs<T>& F, c
   const int w = static_cast<int>(t % s.ext[2]);
   const int v = static_cast<int>((t / s.ext[2]) % s.ext[1]);
   const int u = static_cast<int>(t / (static_cast<int64_t>(s.ext[2]) * s.ext[1]));
-  cpmlPoint<T, IsE>(g, F, s, s.lo[0] + u, s.lo[1] + v, s.lo[2] + w, t);
+  cpmlPoint<T, IsE>(g, F, s, s.lo[0] + u, s.lo[1] + v, s.lo[2] + w, 2 * t);
 }
 
 template <class T, bool IsE>
@@ -578,7 +578,8 @@ __device__ __forceinline__ void cpmlFacePoint(const Grid& g, const FieldPtrs<T>&
   } else {
     return;
   }
-  const int64_t t = (static_cast<int64_t>(p0 - s.lo[0]) * s.ext[1] + (p1 - s.lo[1])) * s.ext[2] + (p2 - s.lo[2]);
+  const int64_t t =
+      2 * ((static_cast<int64_t>(p0 - s.lo[0]) * s.ext[1] + (p1 - s.lo[1])) * s.ext[2] + (p2 - s.lo[2]));
   cpmlPoint<T, IsE>(g, F, s, p0, p1, p2, t);
 }
 
@@ -599,7 +600,7 @@ __global__ __launch_bounds__(256) void k_cpml_zrest(Grid g, FieldPtrs<T> F, Slab
   const int u = static_cast<int>(t / (static_cast<int64_t>(s.ext[2]) * s.ext[1]));
   const int p0 = s.lo[0] + u, p1 = s.lo[1] + v;
   if (p0 < g.nx && p1 < g.ny && !fr.inX(p0) && !fr.inY(p1)) return;
-  cpmlPoint<T, IsE>(g, F, s, p0, p1, s.lo[2] + w, t);
+  cpmlPoint<T, IsE>(g, F, s, p0, p1, s.lo[2] + w, 2 * t);
 }
 
 enum AdeScheme { kAdeDrude = 0, kAdeDebye = 1, kAdeMLorentz = 2 };
@@ -647,13 +648,12 @@ __device__ __forceinline__ T adeUpdate(const AdeArgs<T>& A, int m, int q, int64_
 // first: the cell's pole currents (and, modified Lorentz, previous currents
 // and previous E) of all components, then the arithmetic of adeUpdate in its
 // order, component by component.  `r[q]`: component q is inside its Yee range
-// (outside it the forward update leaves E and the currents alone).  Up to
-// kAdeFastPoles poles (a uniform bound: the unused slots are never loaded).
+// (outside it the forward update leaves E and the currents alone).  Up to P
+// poles (a uniform bound: the unused slots are never loaded).
 constexpr int kAdeFastPoles = 4;
-template <class T, int S>
+template <class T, int S, int P = kAdeFastPoles>
 __device__ __forceinline__ void adeCell(const AdeArgs<T>& A, int m, int64_t idx, const bool r[3], const T cur[3],
                                         const T en[3], T out[3]) {
-  constexpr int P = kAdeFastPoles;
   const int np = A.poles;
   const T* c = A.tab + static_cast<int64_t>(m) * A.stride;
   T jv[3][P], jpv[3][P], ep[3];

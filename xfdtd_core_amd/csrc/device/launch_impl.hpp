@@ -533,6 +533,20 @@ void StepLaunch<T>::step(hipStream_t s, const Grid& g, const FieldPtrs<T>& A, co
   launchStep<T>(s, g, A, B, C, SH, SE, ichunk);
 }
 
+template <class T, class Coef, bool NT, int TK, int TJ, int P>
+void launchHalfAde(hipStream_t s, const Grid& g, const FieldPtrs<T>& F, const Coef& C, const HalfArgs<T>& a,
+                   const SweepMap& m, int64_t t) {
+  const dim3 grid(static_cast<unsigned>(m.nbx * m.nby * m.nbz)), block(TK, TJ);
+  if (a.scheme == kAdeDrude)
+    hipLaunchKernelGGL((k_half<T, Coef, true, kAdeDrude, NT, TK, TJ, P>), grid, block, 0, s, g, F, C, a.ade, a.slabs,
+                       a.events, m, a.ichunk, t);
+  else if (a.scheme == kAdeDebye)
+    hipLaunchKernelGGL((k_half<T, Coef, true, kAdeDebye, NT, TK, TJ, P>), grid, block, 0, s, g, F, C, a.ade, a.slabs,
+                       a.events, m, a.ichunk, t);
+  else
+    hipLaunchKernelGGL((k_half<T, Coef, true, kAdeMLorentz, NT, TK, TJ, P>), grid, block, 0, s, g, F, C, a.ade,
+                       a.slabs, a.events, m, a.ichunk, t);
+}
 template <class T, class Coef, bool NT, int TK, int TJ>
 void launchHalf(hipStream_t s, const Grid& g, const FieldPtrs<T>& F, const Coef& C, const HalfArgs<T>& a, bool is_e,
                 int64_t t) {
@@ -544,15 +558,10 @@ void launchHalf(hipStream_t s, const Grid& g, const FieldPtrs<T>& F, const Coef&
   else if (a.scheme < 0)
     hipLaunchKernelGGL((k_half<T, Coef, true, -1, NT, TK, TJ>), grid, block, 0, s, g, F, C, a.ade, a.slabs, a.events, m,
                        a.ichunk, t);
-  else if (a.scheme == kAdeDrude)
-    hipLaunchKernelGGL((k_half<T, Coef, true, kAdeDrude, NT, TK, TJ>), grid, block, 0, s, g, F, C, a.ade, a.slabs,
-                       a.events, m, a.ichunk, t);
-  else if (a.scheme == kAdeDebye)
-    hipLaunchKernelGGL((k_half<T, Coef, true, kAdeDebye, NT, TK, TJ>), grid, block, 0, s, g, F, C, a.ade, a.slabs,
-                       a.events, m, a.ichunk, t);
+  else if (a.ade.poles <= 2)
+    launchHalfAde<T, Coef, NT, TK, TJ, 2>(s, g, F, C, a, m, t);
   else
-    hipLaunchKernelGGL((k_half<T, Coef, true, kAdeMLorentz, NT, TK, TJ>), grid, block, 0, s, g, F, C, a.ade, a.slabs,
-                       a.events, m, a.ichunk, t);
+    launchHalfAde<T, Coef, NT, TK, TJ, kAdeFastPoles>(s, g, F, C, a, m, t);
 }
 template <class T, class Coef>
 void launchHalfTile(hipStream_t s, const Grid& g, const FieldPtrs<T>& F, const Coef& C, const HalfArgs<T>& a,

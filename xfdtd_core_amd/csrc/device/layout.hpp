@@ -114,6 +114,12 @@ struct CoefPtrs {
   __device__ __forceinline__ Raw raw(int q, int64_t idx) const {
     return Raw{ldOwn<NT>(c[3 * q] + idx), ldOwn<NT>(c[3 * q + 1] + idx), ldOwn<NT>(c[3 * q + 2] + idx)};
   }
+  // the same at a uniform base u and the lane's offset e (scalar base addressing)
+  template <bool NT = true>
+  __device__ __forceinline__ Raw rawAt(int q, int64_t u, unsigned e) const {
+    return Raw{ldOwn<NT>((c[3 * q] + u) + e), ldOwn<NT>((c[3 * q + 1] + u) + e), ldOwn<NT>((c[3 * q + 2] + u) + e)};
+  }
+  __device__ __forceinline__ void resolveAt(int q, const Raw& r, T& s, T& a, T& b) const { resolve(q, r, s, a, b); }
   __device__ __forceinline__ void resolve(int, const Raw& r, T& s, T& a, T& b) const {
     s = r.s;
     a = r.a;
@@ -146,6 +152,19 @@ struct ClassCoef {
   template <bool NT = true>
   __device__ __forceinline__ Raw raw(int q, int64_t idx) const {
     return Raw{static_cast<int>(ldOwn<NT>(id[q] + idx))};
+  }
+  // the same at a uniform base u and the lane's offset e (scalar base
+  // addressing); a table stays below 4 GB
+  template <bool NT = true>
+  __device__ __forceinline__ Raw rawAt(int q, int64_t u, unsigned e) const {
+    return Raw{static_cast<int>(ldOwn<NT>((id[q] + u) + e))};
+  }
+  __device__ __forceinline__ void resolveAt(int q, const Raw& r, T& s, T& a, T& b) const {
+    const T* e = reinterpret_cast<const T*>(reinterpret_cast<const char*>(tab[q]) +
+                                            static_cast<unsigned>(r.id) * static_cast<unsigned>(3 * sizeof(T)));
+    s = e[0];
+    a = e[1];
+    b = e[2];
   }
   __device__ __forceinline__ void resolve(int q, const Raw& r, T& s, T& a, T& b) const {
     const T* e = tab[q] + 3 * r.id;
@@ -258,7 +277,10 @@ struct SlabArgs {
   int extB[2];       // component B extent along (a, b)
   int fieldA, fieldB, dualA, dualB;  // field ids (0..5)
   int64_t stride_c;  // padded-layout stride of the main axis
-  const T* cpsiA;    // box-local layout, k fastest
+  // psi and c_psi in the box layout, k fastest, the components' values of a
+  // point side by side (B = A + 1): point (u, v, w) of the box at
+  // 2 ((u ext[1] + v) ext[2] + w)
+  const T* cpsiA;
   const T* cpsiB;
   T* psiA;
   T* psiB;
@@ -278,7 +300,7 @@ struct CpmlList {
 // for its whole i-march, so it lies in at most one such slab and its layer
 // coefficients are loaded once; only psi and c_psi are read per cell, and the
 // field and dual values come from the sweep's registers.  The slab spans the
-// whole x/y range (box-local psi index t = (i * ext1 + j) * ext2 + k - klo)
+// whole x/y range (psi index t = 2 ((i * ext1 + j) * ext2 + k - klo))
 // and both of its components cover every sweep point (i < nx, j < ny) of its
 // layers [klo, khi); the far planes i = nx, j = ny (k_cpml_faces) and, in
 // FP64, the frame (ZFrame, k_cpml_zrest) are left to a launch of their own.

@@ -26,7 +26,8 @@ constexpr int kLineSegments = 32;    // record segments per half whose addends a
 constexpr int kLineAhead = 64;       // steps whose addends LDS holds
 constexpr int kLineExtra = 64;       // corrected points of the column (0, 1), per field, held in LDS
 
-// The z slab's component on the line: Ex (Hy) corrected from Hy (Ex).
+// The z slab's component on the line, Ex (Hy) corrected from Hy (Ex): every
+// other value of the slab's c_psi and psi.
 template <class T>
 struct LineSlab {
   int lo, n;
@@ -173,12 +174,12 @@ __global__ __launch_bounds__(kLineThreads) void k_line(Coef K, LineArgs<T> a, in
     const int w = q < m0 ? q : q - m0;
     T* se4 = slab + 4 * q;
     T* sh4 = slab + 4 * (cells + q);
-    se4[0] = E.psi[w];
-    se4[1] = E.c[w];
+    se4[0] = E.psi[2 * w];
+    se4[1] = E.c[2 * w];
     se4[2] = E.ca[w];
     se4[3] = E.cb[w];
-    sh4[0] = H.psi[w];
-    sh4[1] = H.c[w];
+    sh4[0] = H.psi[2 * w];
+    sh4[1] = H.c[2 * w];
     sh4[2] = H.ca[w];
     sh4[3] = H.cb[w];
   }
@@ -287,8 +288,8 @@ __global__ __launch_bounds__(kLineThreads) void k_line(Coef K, LineArgs<T> a, in
   }
   for (int q = tid; q < cells; q += nth) {
     const int w = q < m0 ? q : q - m0;
-    a.e[q < m0 ? 0 : 1].psi[w] = slab[4 * q];
-    a.h[q < m0 ? 0 : 1].psi[w] = slab[4 * (cells + q)];
+    a.e[q < m0 ? 0 : 1].psi[2 * w] = slab[4 * q];
+    a.h[q < m0 ? 0 : 1].psi[2 * w] = slab[4 * (cells + q)];
   }
 }
 

@@ -2,8 +2,7 @@
 // slab's parameters travel as kernel arguments (scalar loads), and a point's
 // membership is the AND of per-axis masks, uniform over a plane (i), a row
 // (j) or fixed over a lane's march (k), so points outside every slab cost
-// one test.  Used by the two sweeps (every slab, in boundary order) and by
-// the single-pass step.
+// one test.  Used by the single-pass step.
 #pragma once
 
 #include "layout.hpp"
@@ -80,7 +79,7 @@ __device__ __forceinline__ void stepSlabs(const StepSlabs<T>& L, uint32_t mu, ui
     const StepSlab<T>& S = L.s[n];
     const int u = i - S.lo[0], v = j - S.lo[1], w = k - S.lo[2];
     const int c = S.axis, a = c == 2 ? 0 : c + 1, b = c == 0 ? 2 : c - 1;
-    const int64_t t = (static_cast<int64_t>(u) * S.ext[1] + v) * S.ext[2] + w;
+    const int64_t t = 2 * ((static_cast<int64_t>(u) * S.ext[1] + v) * S.ext[2] + w);
     const int layer = pick3(c, i, j, k) - S.start;
     const T ca = S.ca[layer], cb = S.cb[layer];
     const int pa = pick3(a, i, j, k), pb = pick3(b, i, j, k);

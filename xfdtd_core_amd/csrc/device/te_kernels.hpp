@@ -31,7 +31,8 @@ __device__ __forceinline__ void teTile(const Grid& g, const FieldPtrs<T>& F, con
   T* __restrict__ ez = F.f[2];
   T* __restrict__ hx = F.f[3];
   T* __restrict__ hy = F.f[4];
-  // psi boxes span both entries of k (nz + 1 = 2); only k = 0 moves
+  // psi boxes span both entries of k (nz + 1 = 2) and hold both components;
+  // one of each moves
   const bool inY0 = H.n[1] > 0 && j >= H.s[1][0].lo && j < H.s[1][0].hi;
   const bool inY1 = H.n[1] > 1 && j >= H.s[1][1].lo && j < H.s[1][1].hi;
   const bool inY = inY0 || inY1;
@@ -45,10 +46,10 @@ __device__ __forceinline__ void teTile(const Grid& g, const FieldPtrs<T>& F, con
     const int l = j - (inY1 ? Y1.lo : Y0.lo), n = inY1 ? Y1.hi - Y1.lo : Y0.hi - Y0.lo;
     yca = (inY1 ? Y1.ca : Y0.ca)[l];
     ycb = (inY1 ? Y1.cb : Y0.cb)[l];
-    ystep = 2 * n;
-    const int64_t y = i0 * ystep + 2 * l;
-    yc = (IsE ? (inY1 ? Y1.cA : Y0.cA) : (inY1 ? Y1.cB : Y0.cB)) + y;
-    yp = (IsE ? (inY1 ? Y1.pA : Y0.pA) : (inY1 ? Y1.pB : Y0.pB)) + y;
+    ystep = 4 * n;
+    const int64_t y = i0 * ystep + 4 * l;
+    yc = (inY1 ? Y1.c : Y0.c) + y + (IsE ? 0 : 1);
+    yp = (inY1 ? Y1.psi : Y0.psi) + y + (IsE ? 0 : 1);
   }
   int64_t u = i0 * pl;
   // E: Hy of row i - 1; H: Ez of row i (carried along the march)
@@ -81,10 +82,10 @@ __device__ __forceinline__ void teTile(const Grid& g, const FieldPtrs<T>& F, con
     if (inX) {  // E: component B (Ez), H: component A (Hy)
       xca = X.ca[i - X.lo];
       xcb = X.cb[i - X.lo];
-      const int64_t x = (static_cast<int64_t>(i - X.lo) * g.NY + j) * 2;
-      xpp = (IsE ? X.pB : X.pA) + x;
+      const int64_t x = (static_cast<int64_t>(i - X.lo) * g.NY + j) * 4 + (IsE ? 1 : 0);
+      xpp = X.psi + x;
       xp = *xpp;
-      xc = (IsE ? X.cB : X.cA)[x];
+      xc = X.c[x];
     }
     if (inY) {
       yv = *yp;
