@@ -1,7 +1,7 @@
 """The one-launch half-step (update, CPML slabs, TFSF and lumped corrections,
 probes) against a launch per correction, which the parity tests hold to the
-oracle bitwise: FP64 the same bits, FP32 the same up to the compiler's choice
-of contractions."""
+oracle bitwise: the same bits in FP64 and in FP32, whose sums every kernel writes
+out alike."""
 
 import ctypes
 
@@ -41,14 +41,17 @@ def _box(n, pml=6, faces=("XN", "XP", "YN", "YP", "ZN", "ZP"), tfsf=True):
     return s.spec()
 
 
-def _run(monkeypatch, spec, precision, steps, on, chunk=None):
+def _run(monkeypatch, spec, precision, steps, on, chunk=None, z_inside=False):
     monkeypatch.setenv("XFD_CPML_INSWEEP", "1" if on else "0")
-    monkeypatch.setenv("XFD_CPML_ZFUSED", "0")
+    if z_inside:  # the default: long FP32 rows correct z first, in the sweeps or in the one launch
+        monkeypatch.delenv("XFD_CPML_ZFUSED", raising=False)
+    else:
+        monkeypatch.setenv("XFD_CPML_ZFUSED", "0")
     if chunk:
         monkeypatch.setenv("XFD_ICHUNK", str(chunk))
     sim = native.Simulation(spec, precision)
     sim.init(steps)
-    assert sim.cpml_fused() == (4 if on else 0)
+    assert sim.cpml_fused() == (4 if on else 2 if z_inside else 0)
     return sim
 
 
@@ -56,12 +59,7 @@ def _compare(a, b, precision, label):
     for f in FIELDS:
         x, y = a.field(f), b.field(f)
         assert np.abs(y).max() > 0
-        if precision == "f64":
-            np.testing.assert_array_equal(x, y, err_msg=f"{label} {f}")
-        else:
-            # each step rounds a few times at 6e-8; the two runs' roundings
-            # differ in ~50 steps, far below 1e-4 of the field's norm
-            assert np.linalg.norm(x - y) <= 1e-4 * np.linalg.norm(y), (label, f)
+        np.testing.assert_array_equal(x, y, err_msg=f"{label} {precision} {f}")
 
 
 # nz around the 64- and 128-lane tiles, ny off the 4-row tile, nx off the chunk
@@ -79,14 +77,20 @@ def test_half_step_matches_separate_launches(monkeypatch, n, chunk, precision):
     _compare(a, b, precision, f"{n} {chunk}")
     for m in range(a.monitor_count()):
         for x, y in zip(a.monitor_records(m), b.monitor_records(m)):
-            if precision == "f64":
-                np.testing.assert_array_equal(x, y)
-            else:
-                # a probe outside the TFSF box sees what is left of waves that
-                # cancel, so its rounding is relative to the component's peak:
-                # at most 8 roundings of 6e-8 a step in each run, 50 steps
-                peak = np.abs(b.field(("EZ", "HY", "EX")[m])).max()
-                assert np.abs(x - y).max() <= 2 * 50 * 8 * 6e-8 * peak
+            np.testing.assert_array_equal(x, y)
+
+
+# FP32 rows of three k-tiles and up: the z corrections precede the x and y ones
+@pytest.mark.parametrize("faces", [("XN", "XP", "YN", "YP", "ZN", "ZP"), ("ZN", "ZP", "YP", "YN", "XN", "XP"),
+                                   ("YN", "ZP", "XP", "XN")])
+def test_half_step_order_of_long_fp32_rows(monkeypatch, faces):
+    spec, steps = _box((22, 21, 140), faces=faces, tfsf=len(faces) == 6), 60
+    a = _run(monkeypatch, spec, "f32", steps, True, z_inside=True)
+    b = _run(monkeypatch, spec, "f32", steps, False, z_inside=True)
+    for sim in (a, b):
+        sim.advance(0, steps)
+        sim.finish()
+    _compare(a, b, "f32", str(faces))
 
 
 # the slabs' order decides which correction a point of two slabs adds first
@@ -166,13 +170,11 @@ def test_plane_half_step(monkeypatch, nx, ny, chunk, faces, precision):
         sim.finish()
         runs.append(sim)
     a, b = runs
-    # FP32 as above, relative to the incident wave (1 V/m)
-    tol = 0 if precision == "f64" else 2 * steps * 8 * 6e-8
     for f in FIELDS:
-        assert np.abs(a.field(f) - b.field(f)).max() <= tol * (1 if f[0] == "E" else 1 / 376), f
+        np.testing.assert_array_equal(a.field(f), b.field(f), err_msg=f)
     for m in range(a.monitor_count()):
         for x, y in zip(a.monitor_records(m), b.monitor_records(m)):
-            assert np.abs(x - y).max() <= tol * (1 / 376 if m == 1 else 1), m
+            np.testing.assert_array_equal(x, y)
     assert np.abs(b.field("EZ")).max() > 0
 
 
@@ -192,3 +194,29 @@ def test_plane_half_step_after_writes(monkeypatch):
         runs.append(sim)
     _te = [np.abs(runs[0].field(f) - runs[1].field(f)).max() for f in FIELDS]
     assert _te == [0] * 6
+
+
+@pytest.mark.parametrize("on", [True, False])
+def test_fp32_keeps_the_field_product_unrounded(monkeypatch, on):
+    """E = s E + a d with s != 1: the product s E, the larger one, is not rounded
+    by itself, so one step is within the one rounding of its result (half a unit
+    in the last place) and that of a d (2^-24 of it)."""
+    monkeypatch.setenv("XFD_CPML_INSWEEP", "1" if on else "0")
+    n, rng = (9, 11, 70), np.random.default_rng(1)
+    ext = {c: tuple(m + (1 if (q != "xyz".index(c[0]) if c[1] == "e" else q == "xyz".index(c[0])) else 0)
+                    for q, m in enumerate(n)) for c in ("xe", "ye", "ze", "xh", "yh", "zh")}
+    f32 = lambda v: v.astype(np.float32).astype(np.float64)  # noqa: E731
+    coeffs = {name: np.full(ext[name[2] + name[1]], 1.0 if name[1] == name[3] else 0.0) for name in native.COEFF_NAMES}
+    s, a = (f32(rng.choice(v, ext["xe"])) for v in ((0.7, 0.9, 0.99), (0.013, 0.021)))
+    coeffs["cexe"], coeffs["cexhy"] = s, a
+    ctx = native.Context(coeffs, "f32")
+    e, h = f32(rng.standard_normal(ext["xe"])), f32(rng.standard_normal(ext["yh"]))
+    ctx.write("EX", e)
+    ctx.write("HY", h)
+    ctx.step(0, 1)
+    got = ctx.read("EX")[:, 1:-1, 1:-1]
+    ad = a[:, 1:-1, 1:-1] * f32(np.diff(h, axis=2))[:, 1:-1]
+    want = s[:, 1:-1, 1:-1] * e[:, 1:-1, 1:-1] + ad
+    unit = np.spacing(np.maximum(np.abs(got), np.abs(want)).astype(np.float32))
+    assert (np.abs(got - want) <= 0.5 * unit + 2.0**-24 * np.abs(ad)).all()
+    assert np.abs(got - e[:, 1:-1, 1:-1]).max() > 0

@@ -1,6 +1,5 @@
 """1D grids stepped many times per launch against a launch per correction,
-which the low-dimension tests hold to the oracle: FP64 the same bits, FP32 up to
-the compiler's choice of contractions."""
+which the low-dimension tests hold to the oracle: the same bits in FP64 and FP32."""
 
 import numpy as np
 import pytest
@@ -54,13 +53,9 @@ def test_line_steps_match_separate_launches(monkeypatch, nz, tfsf, faces, precis
         sim.finish()
         sims.append(sim)
     a, b = sims
-    # FP32: at most 8 roundings of 6e-8 a step in each run, relative to the
-    # incident wave (1 V/m), whose parts cancel outside the TFSF region
-    tol = 0 if precision == "f64" else 2 * steps * 8 * 6e-8
     for f in ("EX", "EY", "EZ", "HX", "HY", "HZ"):
-        x, y = a.field(f), b.field(f)
-        assert np.abs(x - y).max() <= tol * (1 if f[0] == "E" else 1 / 376), f
+        np.testing.assert_array_equal(a.field(f), b.field(f), err_msg=f)
     for m in range(a.monitor_count()):
         for x, y in zip(a.monitor_records(m), b.monitor_records(m)):
-            assert np.abs(x - y).max() <= tol * (1 / 376 if m == 1 else 1), m
+            np.testing.assert_array_equal(x, y)
     assert np.abs(b.field("EX")).max() > 0

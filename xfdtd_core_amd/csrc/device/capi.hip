@@ -328,6 +328,8 @@ struct xfd_ctx {
   // each half-step (update, every CPML slab, records, point probes) as one
   // launch (k_half), with its records and probes by tile
   bool half = false;
+  // the z slabs' corrections come before the x / y slabs' (FP32 rounding only)
+  bool z_first = false;
   int half_tk = 64, half_tj = 4, half_chunk = 4;  // tile: k-lanes x j-rows x i-planes
   // the far planes i = nx, j = ny, k = nz hold zeros, which their slab
   // corrections keep (they draw on each other only), so no launch visits them
@@ -834,6 +836,9 @@ void halfSetup(xfd_ctx& c, const std::vector<xfd::Record>& re, const std::vector
            !is("XFD_CPML_INSWEEP", '0') && !is("XFD_STEP_FUSED", '0') && !is("XFD_CPML_FUSED", '1') &&
            !is("XFD_CPML_ZFUSED", '1');
   if (!c.half) return;
+  // FP32 rows on which the sweeps would take the z slabs (zfused) keep the order
+  // that has: results do not depend on which of the two paths a grid takes.
+  c.z_first = c.zfused;
   c.fused = false;
   c.n_fused = 0;
   c.zfused = false;
@@ -1615,6 +1620,10 @@ std::vector<xfd::HalfSlabs<T>> halfSlabs(xfd_ctx& c, bool is_e) {
   xfd::HalfSlabs<T>& H = v[0];
   int slab[3][2];
   require(slabsByAxis(c, H.n, slab, H.swap), "CPML slab order");
+  if (c.z_first) {  // component 0: y then z in axis order; 1: z then x
+    H.swap[0] = 1;
+    H.swap[1] = 0;
+  }
   for (int ax = 0; ax < 3; ++ax)
     for (int q = 0; q < H.n[ax]; ++q) {
       const auto s = slabArgs<T>(*c.slabs[slab[ax][q]], is_e);

@@ -100,21 +100,11 @@ __device__ __forceinline__ SlabVals<T> slabLoad(const T* c, const T* psi, int64_
   return SlabVals<T>{p.a, p.b, q.a, q.b};
 }
 
-// a b + c: fused in FP32, two roundings in FP64 (the reference's).  Explicit,
-// with contraction off around it, so that every instance of the kernel (dense
-// or class-id coefficients, either tile) rounds alike.
-__device__ __forceinline__ float mulAdd(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
-__device__ __forceinline__ double mulAdd(double a, double b, double c) {
-#pragma clang fp contract(off)
-  return a * b + c;
-}
-
 // psi = b psi + a d for both components of a slab point, stored.
 template <class T>
 __device__ __forceinline__ void slabStore(T* psi, int64_t u, unsigned e, SlabVals<T>& v, T ca, T cb, T dA, T dB) {
-#pragma clang fp contract(off)
-  v.pA = mulAdd(ca, dA, cb * v.pA);
-  v.pB = mulAdd(ca, dB, cb * v.pB);
+  v.pA = sumTwo(cb, v.pA, ca, dA);
+  v.pB = sumTwo(cb, v.pB, ca, dB);
   (reinterpret_cast<SlabPair<T>*>(psi) + u)[e] = SlabPair<T>{v.pA, v.pB};
 }
 
@@ -280,9 +270,9 @@ __device__ __forceinline__ void halfTile(const Grid g, const FieldPtrs<T> F, con
     const T y0 = IsE ? a0 - L.j0 : L.j0 - a0, y2 = IsE ? b2 - L.j2 : L.j2 - b2;
     const T z0 = IsE ? a0 - L.k0 : L.k0 - a0, z1 = IsE ? b1 - L.k1 : L.k1 - b1;
     // component 0: d1 along z, d2 along y; 1: d2 along x, d0 along z; 2: d0 along y, d1 along x
-    const T w0 = mulAdd(r0, y2, mulAdd(p0, z1, s0 * o0));
-    const T w1 = mulAdd(r1, z0, mulAdd(p1, x2, s1 * o1));
-    const T w2 = mulAdd(r2, x1, mulAdd(p2, y0, s2 * o2));
+    const T w0 = IsE ? sumE(s0, o0, p0, z1, r0, y2) : sumH(s0, o0, p0, z1, r0, y2);
+    const T w1 = IsE ? sumE(s1, o1, p1, x2, r1, z0) : sumH(s1, o1, p1, x2, r1, z0);
+    const T w2 = IsE ? sumE(s2, o2, p2, y0, r2, x1) : sumH(s2, o2, p2, y0, r2, x1);
     T v0 = w0, v1 = w1, v2 = w2;
     if (IsE) {
       const bool r[3] = {jk, i >= 1 && k >= 1, i >= 1 && j >= 1};

@@ -181,12 +181,12 @@ __device__ __forceinline__ void zStore(const ZCpml<T>& Z, const ZLane<T>& L, con
   if (v.act) {
     const ZSlab<T>& s0 = Z.z[0];
     const ZSlab<T>& s1 = Z.z[1];
-    const T psiA = L.cb * v.pA + L.ca * dA;
-    const T psiB = L.cb * v.pB + L.ca * dB;
+    const T psiA = sumTwo(L.cb, v.pA, L.ca, dA);
+    const T psiB = sumTwo(L.cb, v.pB, L.ca, dB);
     (L.sel ? s1.psiA : s0.psiA)[L.t] = psiA;
     (L.sel ? s1.psiB : s0.psiB)[L.t] = psiB;
-    vA += v.cA * psiA;
-    vB += v.cB * psiB;
+    vA = mulAdd(v.cA, psiA, vA);
+    vB = mulAdd(v.cB, psiB, vB);
   }
 }
 
@@ -225,11 +225,11 @@ __device__ __forceinline__ void sweepH(const Grid& g, const FieldPtrs<T>& F, con
     const T ez_j = ez[idx + pz], ez_n = ez[idx + pl];
     T s, a, b;
     C.getOwn(3, idx, s, a, b);
-    T vx = s * ldOwn(hx + idx) + a * (ey_k - ey_i) + b * (ez_j - ez_i);
+    T vx = sumH(s, ldOwn(hx + idx), a, ey_k - ey_i, b, ez_j - ez_i);
     C.getOwn(4, idx, s, a, b);
-    T vy = s * ldOwn(hy + idx) + a * (ez_n - ez_i) + b * (ex_k - ex0);
+    T vy = sumH(s, ldOwn(hy + idx), a, ez_n - ez_i, b, ex_k - ex0);
     C.getOwn(5, idx, s, a, b);
-    T vz = s * ldOwn(hz + idx) + a * (ex_j - ex0) + b * (ey_n - ey_i);
+    T vz = sumH(s, ldOwn(hz + idx), a, ex_j - ex0, b, ey_n - ey_i);
     if (Fused && mask)  // A: Hy(x) <- Ez, Hz(y) <- Ex, Hx(z) <- Ey;  B: Hz(x) <- Ey, Hx(y) <- Ez, Hy(z) <- Ex
       cpmlFused(P, mask, i, j, k, vx, vy, vz, ez_n - ez_i, ex_j - ex0, ey_k - ey_i, ey_n - ey_i, ez_j - ez_i,
                 ex_k - ex0);
@@ -302,9 +302,9 @@ __device__ __forceinline__ void sweepE(const Grid& g, const FieldPtrs<T>& F, con
       C.getOwn(0, idx, s, a, b);
       C.getOwn(1, idx, s1, a1, b1);
       C.getOwn(2, idx, s2, a2, b2);
-      const T ux = s * vx + a * (hy0 - hy_k) + b * (hz0 - hz_j);
-      const T uy = s1 * vy + a1 * (hz0 - hz_p) + b1 * (hx0 - hx_k);
-      const T uz = s2 * vz + a2 * (hx0 - hx_j) + b2 * (hy0 - hy_p);
+      const T ux = sumE(s, vx, a, hy0 - hy_k, b, hz0 - hz_j);
+      const T uy = sumE(s1, vy, a1, hz0 - hz_p, b1, hx0 - hx_k);
+      const T uz = sumE(s2, vz, a2, hx0 - hx_j, b2, hy0 - hy_p);
       vx = jk ? ux : vx;
       vy = (i >= 1 && k >= 1) ? uy : vy;
       vz = (i >= 1 && j >= 1) ? uz : vz;
@@ -377,20 +377,20 @@ __global__ __launch_bounds__(256) void k_te_h(Grid g, FieldPtrs<T> F, Coef C) {
   T s, a, b;
   if (TeZero) {
     C.get(3, idx, s, a, b);
-    const T vx = s * F.f[3][idx] + b * (ez[idx + pz] - ez[idx]);
+    const T vx = sumTwo(s, F.f[3][idx], b, ez[idx + pz] - ez[idx]);
     T s4, a4, b4;
     C.get(4, idx, s4, a4, b4);
-    const T vy = s4 * F.f[4][idx] + a4 * (ez[idx + pl] - ez[idx]);
+    const T vy = sumTwo(s4, F.f[4][idx], a4, ez[idx + pl] - ez[idx]);
     F.f[3][idx] = vx;
     F.f[4][idx] = vy;
     return;
   }
   C.get(3, idx, s, a, b);
-  const T vx = s * F.f[3][idx] + a * (ey[idx + g.kz] - ey[idx]) + b * (ez[idx + pz] - ez[idx]);
+  const T vx = sumE(s, F.f[3][idx], a, ey[idx + g.kz] - ey[idx], b, ez[idx + pz] - ez[idx]);
   C.get(4, idx, s, a, b);
-  const T vy = s * F.f[4][idx] + a * (ez[idx + pl] - ez[idx]) + b * (ex[idx + g.kz] - ex[idx]);
+  const T vy = sumE(s, F.f[4][idx], a, ez[idx + pl] - ez[idx], b, ex[idx + g.kz] - ex[idx]);
   C.get(5, idx, s, a, b);
-  const T vz = s * F.f[5][idx] + a * (ex[idx + pz] - ex[idx]) + b * (ey[idx + pl] - ey[idx]);
+  const T vz = sumE(s, F.f[5][idx], a, ex[idx + pz] - ex[idx], b, ey[idx + pl] - ey[idx]);
   F.f[3][idx] = vx;
   F.f[4][idx] = vy;
   F.f[5][idx] = vz;
@@ -409,7 +409,7 @@ __global__ __launch_bounds__(256) void k_te_e(Grid g, FieldPtrs<T> F, Coef C) {
   const T* __restrict__ hy = F.f[4];
   T s, a, b;
   C.get(2, idx, s, a, b);
-  F.f[2][idx] = s * F.f[2][idx] + a * (hx[idx] - hx[idx - pz]) + b * (hy[idx] - hy[idx - pl]);
+  F.f[2][idx] = sumE(s, F.f[2][idx], a, hx[idx] - hx[idx - pz], b, hy[idx] - hy[idx - pl]);
 }
 
 // BasicUpdatorTEM::updateE (src/updator/basic_updator.cpp:90-109) on a 1D
@@ -423,7 +423,7 @@ __global__ __launch_bounds__(256) void k_tem_e(Grid g, FieldPtrs<T> F, Coef C) {
   const T* __restrict__ hy = F.f[4];
   T s, a, b;
   C.get(0, idx, s, a, b);
-  F.f[0][idx] = s * F.f[0][idx] + a * (hy[idx] - hy[idx - 1]) + T(0) * (T(0) - T(0));
+  F.f[0][idx] = sumTwo(s, F.f[0][idx], a, hy[idx] - hy[idx - 1]) + T(0);  // the reference adds its zero b term
 }
 
 // Single-cell time series (FieldTimeMonitor sampling): one launch per step
@@ -499,13 +499,15 @@ __device__ __forceinline__ void cpmlPoint(const Grid& g, const FieldPtrs<T>& F, 
   const Pair c_psi = ldOwn(reinterpret_cast<const Pair*>(s.cpsiA + t));
   if (inA) {
     const T* dual = F.f[s.dualB];
-    psi.x = IsE ? cb * psi.x + ca * (dual[idx] - dual[q]) : cb * psi.x + ca * (dual[q] - dual[idx]);
-    F.f[s.fieldA][idx] += c_psi.x * psi.x;
+    psi.x = sumTwo<T>(cb, psi.x, ca, IsE ? dual[idx] - dual[q] : dual[q] - dual[idx]);
+    T* f = F.f[s.fieldA];
+    f[idx] = mulAdd(c_psi.x, psi.x, f[idx]);
   }
   if (inB) {
     const T* dual = F.f[s.dualA];
-    psi.y = IsE ? cb * psi.y + ca * (dual[idx] - dual[q]) : cb * psi.y + ca * (dual[q] - dual[idx]);
-    F.f[s.fieldB][idx] += c_psi.y * psi.y;
+    psi.y = sumTwo<T>(cb, psi.y, ca, IsE ? dual[idx] - dual[q] : dual[q] - dual[idx]);
+    T* f = F.f[s.fieldB];
+    f[idx] = mulAdd(c_psi.y, psi.y, f[idx]);
   }
   stOwn(reinterpret_cast<Pair*>(s.psiA + t), psi);
 }
@@ -745,9 +747,9 @@ __device__ __forceinline__ void sweepEAde(const Grid& g, const FieldPtrs<T>& F, 
     C.getOwn(0, idx, s0, a0, b0);
     C.getOwn(1, idx, s1, a1, b1);
     C.getOwn(2, idx, s2, a2, b2);
-    const T en[3] = {s0 * cur[0] + a0 * (hy0 - hy_k) + b0 * (hz0 - hz_j),
-                     s1 * cur[1] + a1 * (hz0 - hz_p) + b1 * (hx0 - hx_k),
-                     s2 * cur[2] + a2 * (hx0 - hx_j) + b2 * (hy0 - hy_p)};
+    const T en[3] = {sumE(s0, cur[0], a0, hy0 - hy_k, b0, hz0 - hz_j),
+                     sumE(s1, cur[1], a1, hz0 - hz_p, b1, hx0 - hx_k),
+                     sumE(s2, cur[2], a2, hx0 - hx_j, b2, hy0 - hy_p)};
     const bool r[3] = {jk, i >= 1 && k >= 1, i >= 1 && j >= 1};
     T v[3];
     if (m < 0) {
@@ -958,6 +960,22 @@ __global__ __launch_bounds__(256) void k_far_reduce(int na, int chunks, const do
 // Lumped-element and TFSF corrections: one thread per corrected cell applies
 // that cell's records in the reference's corrector order.  `state` holds the
 // inductor currents (one slot per inductor edge).
+// A record's sums are double; FP32 grids fuse them (then round to float), FP64
+// grids round twice, as the reference.
+template <class T>
+__device__ __forceinline__ double recordAdd(double a, double b, double c) {
+#pragma clang fp contract(off)
+  return sizeof(T) == sizeof(float) ? __builtin_fma(a, b, c) : a * b + c;
+}
+
+// A TFSF record's incident value in table row `row`: TFSFCorrector::exInc..hzInc
+// (tfsf_corrector.cpp:16-122).
+template <class T>
+__device__ __forceinline__ double recordInc(const Record& R, const double* row) {
+#pragma clang fp contract(off)
+  return R.tr * recordAdd<T>(R.omw, row[0], R.w * row[1]);
+}
+
 template <class T>
 __device__ __forceinline__ T recordRun(T value, const Record* __restrict__ rec, int64_t r0, int64_t r1,
                                        const double* __restrict__ pool, T* __restrict__ state, int64_t t) {
@@ -965,20 +983,17 @@ __device__ __forceinline__ T recordRun(T value, const Record* __restrict__ rec, 
   for (int64_t r = r0; r < r1; ++r) {
     const Record R = rec[r];
     if (R.kind == 0) {
-      // TFSFCorrector::exInc..hzInc (tfsf_corrector.cpp:16-122) times the
-      // signed coefficient (tfsf_corrector.h:216-225)
-      const double* row = pool + R.pool + t * R.row;
-      const double inc = R.tr * (R.omw * row[0] + R.w * row[1]);
-      acc = acc + inc * R.coef;
+      // times the signed coefficient (tfsf_corrector.h:216-225)
+      acc = recordAdd<T>(recordInc<T>(R, pool + R.pool + t * R.row), R.coef, acc);
     } else if (R.kind == 1) {
       // Voltage/CurrentSourceCorrector: E += coff * w[t]
-      acc = acc + R.coef * pool[R.pool + t];
+      acc = recordAdd<T>(R.coef, pool[R.pool + t], acc);
     } else {
       // InductorCorrector::correctE: E += cecjc * J, then J += cjcec * E
       const double j = static_cast<double>(state[R.pool]);
-      acc = acc + R.coef * j;
+      acc = recordAdd<T>(R.coef, j, acc);
       if (sizeof(T) == sizeof(float)) acc = static_cast<double>(static_cast<T>(acc));
-      state[R.pool] = static_cast<T>(j + R.w * acc);
+      state[R.pool] = static_cast<T>(recordAdd<T>(R.w, acc, j));
     }
     if (sizeof(T) == sizeof(float)) acc = static_cast<double>(static_cast<T>(acc));
   }

@@ -70,12 +70,14 @@ struct LineArgs {
 };
 
 // True where a segment is one TFSF or waveform record: its addend does not
-// depend on the fields.
+// depend on the fields.  The part without the record's coefficient is computed
+// ahead, so that the sum at the point rounds as recordRun's.
 __device__ __forceinline__ bool plainSegment(const Record* rec, const int64_t* seg, int64_t s) {
   return seg[s + 1] - seg[s] == 1 && rec[seg[s]].kind != 2;
 }
 
-// The addends of every plain segment for steps [t0, t0 + n), in step order:
+// The addends of every plain segment, without their coefficients, for steps [t0,
+// t0 + n), in step order:
 // out[s * kLineSteps + t - t0].  The tables hold a step's row kilobytes from
 // the next one's, so read inside the step they cost trips to memory that the
 // whole line waits for; k_line takes the addends through LDS, kLineAhead steps
@@ -85,19 +87,19 @@ __global__ __launch_bounds__(256) void k_line_addends(const Record* __restrict__
                                                       const int64_t* __restrict__ seg, int64_t nseg,
                                                       const double* __restrict__ pool, int64_t t0, int64_t n,
                                                       double* __restrict__ out) {
-#pragma clang fp contract(off)
   const int64_t q = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   const int64_t s = blockIdx.y;
   if (q >= n || !plainSegment(rec, seg, s)) return;
   const Record R = rec[seg[s]];
   const double* row = pool + R.pool + (t0 + q) * R.row;
-  out[s * kLineSteps + q] = R.kind == 0 ? R.tr * (R.omw * row[0] + R.w * row[1]) * R.coef : R.coef * row[0];
+  out[s * kLineSteps + q] = R.kind == 0 ? recordInc<T>(R, row) : row[0];
 }
 
 // A work-item's records of one half-step; the first one, where plain, without
 // a global access.
 struct LineRecords {
   int r0, r1, at, plain;  // plain: the first segment, or -1
+  double coef;            // its coefficient
 
   template <class T>
   __device__ __forceinline__ void init(const LineEvents<T>& e) {
@@ -105,20 +107,23 @@ struct LineRecords {
     r1 = e.off ? e.off[threadIdx.x + 1] : 0;
     at = 0;
     plain = -1;
+    coef = 0;
     if (r0 < r1 && e.addends) {
       const int s = e.of[r0];
       at = e.loc[s];
-      if (plainSegment(e.rec, e.seg, s)) plain = s;
+      if (plainSegment(e.rec, e.seg, s)) {
+        plain = s;
+        coef = e.rec[e.seg[s]].coef;
+      }
     }
   }
   // corrects the work-item's points of f (LDS) for step t; add: the addends (LDS) of step t
   template <class T>
   __device__ __forceinline__ void apply(T* f, const LineEvents<T>& e, const double* add, const double* pool,
                                         T* state, int64_t t) {
-#pragma clang fp contract(off)
     int r = r0;
     if (plain >= 0) {
-      f[at] = static_cast<T>(static_cast<double>(f[at]) + add[plain * kLineAhead]);
+      f[at] = static_cast<T>(recordAdd<T>(add[plain * kLineAhead], coef, static_cast<double>(f[at])));
       ++r;
     }
     for (; r < r1; ++r) {
@@ -221,7 +226,7 @@ __global__ __launch_bounds__(kLineThreads) void k_line(Coef K, LineArgs<T> a, in
       for (int k = k0[q]; k < hi; k += nth) {
         T* v = base + 4 * ((q ? m0 : 0) + k - lo);
         const T diff = dk < 0 ? d[k] - d[k - 1] : d[k + 1] - d[k];
-        const T psi = mulAdd(v[2], diff, v[3] * v[0]);
+        const T psi = sumTwo(v[3], v[0], v[2], diff);
         v[0] = psi;
         f[k] = mulAdd(v[1], psi, f[k]);
       }
@@ -255,7 +260,7 @@ __global__ __launch_bounds__(kLineThreads) void k_line(Coef K, LineArgs<T> a, in
 #pragma unroll
     for (int c = 0; c < C; ++c) {
       const int k = tid + c * nth;
-      if (k >= 1 && k < nz) ex[k] = mulAdd(ae[c], hy[k] - hy[k - 1], se[c] * ex[k]);
+      if (k >= 1 && k < nz) ex[k] = sumTwo(se[c], ex[k], ae[c], hy[k] - hy[k - 1]);
     }
     if (RE.r0 < RE.r1) RE.apply(ex, a.re, add_e + ahead, a.pool, a.state, t);
     slabs(a.e, ke, slab, ex, hy, -1);

@@ -96,20 +96,20 @@ __device__ __forceinline__ void teTile(const Grid& g, const FieldPtrs<T>& F, con
     // differences along x and y
     const T dx = n1 - c, dy = IsE ? n0 - hxm : n0 - c;
     if (inX) {
-      xp = mulAdd(xca, dx, xcb * xp);
+      xp = sumTwo(xcb, xp, xca, dx);
       *xpp = xp;
     }
     if (inY) {
-      yv = mulAdd(yca, dy, ycb * yv);
+      yv = sumTwo(ycb, yv, yca, dy);
       *yp = yv;
     }
     if (IsE) {
-      T v = mulAdd(b0, dx, mulAdd(a0, dy, s0 * o0));
+      T v = sumE(s0, o0, a0, dy, b0, dx);
       v = i >= 1 && j >= 1 ? v : o0;
       (ez + u)[lane] = addInOrder(v, xc, xp, ycv, yv, H.swap[2]);
     } else {
-      (hx + u)[lane] = mulAdd(ycv, yv, mulAdd(b0, dy, s0 * o0));
-      (hy + u)[lane] = mulAdd(xc, xp, mulAdd(a1, dx, s1 * o1));
+      (hx + u)[lane] = mulAdd(ycv, yv, sumTwo(s0, o0, b0, dy));
+      (hy + u)[lane] = mulAdd(xc, xp, sumTwo(s1, o1, a1, dx));
     }
     c = n1;
     yc += ystep;
