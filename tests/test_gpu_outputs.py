@@ -11,6 +11,8 @@ with the oracle's array of the same scenario (FP64: bitwise for the fields,
 1e-12 for the far-field sums).
 """
 
+import threading
+
 import numpy as np
 import pytest
 
@@ -108,3 +110,30 @@ def test_output_files_match_oracle(tmp_path):
         want = ref.nf2ff_power(0, fi)
         assert abs(power[1, fi] - want) <= 1e-12 * abs(want), (fi, power[1, fi], want)
     dev.close()
+
+
+def test_far_field_calls_from_several_threads():
+    """One finished run asked from four threads for different frequencies and
+    direction counts (so its workspace also grows between them): the bits of
+    the same calls made one after the other."""
+    dev = native.Simulation(_scenario(None), "f64")
+    dev.run(STEPS)
+    asks = [(f % len(FREQS), bool(f & 1), bool(f & 2), np.linspace(0.1, 3.0, n), 0.1 * f)
+            for f, n in enumerate((3, 700, 61, 181))]
+    got = [[] for _ in asks]
+
+    def work(q):
+        f, a_pot, th, theta, phi = asks[q]
+        for _ in range(20):
+            got[q].append(dev.nf2ff_potential(0, f, a_pot, th, theta, phi))
+
+    threads = [threading.Thread(target=work, args=(q,)) for q in range(len(asks))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for (f, a_pot, th, theta, phi), results in zip(asks, got):
+        want = dev.nf2ff_potential(0, f, a_pot, th, theta, phi)
+        assert np.abs(want).max() > 0 and len(results) == 20
+        for r in results:
+            np.testing.assert_array_equal(r, want)

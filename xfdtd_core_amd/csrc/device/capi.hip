@@ -352,7 +352,8 @@ struct xfd_ctx {
 
   // checkpoints of a forward run for the adjoint (xfd_forward_checkpointed)
   DevBuf ckpt;
-  DevBuf far_ws;  // xfd_nf2ff_far_field: inputs, partial sums, result
+  DevBuf far_ws;      // xfd_nf2ff_far_field: inputs, partial sums, result
+  std::mutex far_mu;  // held from the workspace's growth until its result is read
   int64_t ck_interval = 0, ck_nt = 0, ck_bytes = 0;
 
   bool prof = false;
@@ -2859,6 +2860,9 @@ int xfd_nf2ff_far_field(xfd_ctx* c, int32_t n, int32_t f, int32_t na, const doub
     fa.k = k;
     const size_t n_part = static_cast<size_t>(na) * xfd::Launch<double>::farChunks(na) * 8;
     const size_t bytes = (in.size() + n_part + static_cast<size_t>(na) * 8) * sizeof(double);
+    // several host threads may ask one context for different frequencies; the
+    // calls share its stream, so they wait for each other in any case
+    std::lock_guard<std::mutex> lock(c->far_mu);
     if (c->far_ws.bytes < bytes) c->far_ws.alloc(bytes);
     double* dev = c->far_ws.as<double>();
     XFD_HIP(hipMemcpyAsync(dev, in.data(), in.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
