@@ -184,48 +184,9 @@ enum KernelClass {
 const char* kKernelNames[K_COUNT] = {"update_h",  "update_e", "cpml_h", "cpml_e", "records_h",
                                      "records_e", "gather",   "nf2ff",  "step"};
 
-struct DevBuf {
-  void* p = nullptr;
-  size_t bytes = 0;
-  DevBuf() = default;
-  DevBuf(const DevBuf&) = delete;
-  DevBuf& operator=(const DevBuf&) = delete;
-  DevBuf(DevBuf&& o) noexcept : p(o.p), bytes(o.bytes) {
-    o.p = nullptr;
-    o.bytes = 0;
-  }
-  DevBuf& operator=(DevBuf&& o) noexcept {
-    if (this != &o) {
-      reset();
-      p = o.p;
-      bytes = o.bytes;
-      o.p = nullptr;
-      o.bytes = 0;
-    }
-    return *this;
-  }
-  ~DevBuf() {
-    if (p) (void)hipFree(p);
-  }
-  void reset() {
-    if (p) (void)hipFree(p);
-    p = nullptr;
-    bytes = 0;
-  }
-  void alloc(size_t b) {
-    reset();
-    bytes = b;
-    if (b == 0) return;
-    XFD_HIP(hipMalloc(&p, b));
-    XFD_HIP(hipMemset(p, 0, b));
-  }
-  template <class T>
-  T* as() const {
-    return static_cast<T*>(p);
-  }
-};
-
 }  // namespace
+
+#include "dev_buf.hpp"  // uses XFD_HIP
 
 struct xfd_ctx {
   xfd::HostStage::User stage_user;
