@@ -15,6 +15,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 namespace xfd {
 
@@ -165,47 +166,39 @@ template <class T, class Id = uint16_t>
 struct ClassCoef {
   const Id* id[6];
   const T* tab[6];  // 3 values per class
-  __device__ __forceinline__ void get(int q, int64_t idx, T& s, T& a, T& b) const {
-    const T* e = tab[q] + 3 * static_cast<int>(id[q][idx]);
+  // byte offset of class c's entry: 16-bit ids stay within 32 bits, the tables of
+  // 32-bit ids (up to a quarter of the cells) do not
+  using Offset = std::conditional_t<sizeof(Id) == 2, uint32_t, uint64_t>;
+  __host__ __device__ static constexpr Offset entryAt(Id c) {
+    return static_cast<Offset>(c) * static_cast<Offset>(3 * sizeof(T));
+  }
+  __device__ __forceinline__ void entry(int q, Id c, T& s, T& a, T& b) const {
+    const T* e = reinterpret_cast<const T*>(reinterpret_cast<const char*>(tab[q]) + entryAt(c));
     s = e[0];
     a = e[1];
     b = e[2];
   }
+  __device__ __forceinline__ void get(int q, int64_t idx, T& s, T& a, T& b) const { entry(q, id[q][idx], s, a, b); }
   // the same for the cell a sweep owns (its id is read once per pass)
   __device__ __forceinline__ void getOwn(int q, int64_t idx, T& s, T& a, T& b) const {
-    const T* e = tab[q] + 3 * static_cast<int>(ldOwn(id[q] + idx));
-    s = e[0];
-    a = e[1];
-    b = e[2];
+    entry(q, ldOwn(id[q] + idx), s, a, b);
   }
   // split access (a load issued ahead of its use, then its values): the
   // class id, then its table entry
   struct Raw {
-    int id;
+    Id id;
   };
   template <bool NT = true>
   __device__ __forceinline__ Raw raw(int q, int64_t idx) const {
-    return Raw{static_cast<int>(ldOwn<NT>(id[q] + idx))};
+    return Raw{ldOwn<NT>(id[q] + idx)};
   }
-  // the same at a uniform base u and the lane's offset e (scalar base
-  // addressing); a table stays below 4 GB
+  // the same at a uniform base u and the lane's offset e (scalar base addressing)
   template <bool NT = true>
   __device__ __forceinline__ Raw rawAt(int q, int64_t u, unsigned e) const {
-    return Raw{static_cast<int>(ldOwn<NT>((id[q] + u) + e))};
+    return Raw{ldOwn<NT>((id[q] + u) + e)};
   }
-  __device__ __forceinline__ void resolveAt(int q, const Raw& r, T& s, T& a, T& b) const {
-    const T* e = reinterpret_cast<const T*>(reinterpret_cast<const char*>(tab[q]) +
-                                            static_cast<unsigned>(r.id) * static_cast<unsigned>(3 * sizeof(T)));
-    s = e[0];
-    a = e[1];
-    b = e[2];
-  }
-  __device__ __forceinline__ void resolve(int q, const Raw& r, T& s, T& a, T& b) const {
-    const T* e = tab[q] + 3 * r.id;
-    s = e[0];
-    a = e[1];
-    b = e[2];
-  }
+  __device__ __forceinline__ void resolveAt(int q, const Raw& r, T& s, T& a, T& b) const { entry(q, r.id, s, a, b); }
+  __device__ __forceinline__ void resolve(int q, const Raw& r, T& s, T& a, T& b) const { entry(q, r.id, s, a, b); }
 };
 
 // 32-bit class ids, for grids with more distinct triples per component than
@@ -214,6 +207,7 @@ struct ClassCoef {
 // coefficients, and the same branch-free reads.
 template <class T>
 using WideCoef = ClassCoef<T, uint32_t>;
+static_assert(WideCoef<double>::entryAt(200000000u) == 4800000000ull, "a table may pass 4 GB");
 
 // ADE state and per-material coefficients for the dispersive E update.
 // `mat` is a per-cell material id in the padded layout (-1: plain update);
