@@ -1536,7 +1536,7 @@ xfd::ZSlab<T> zSlab(const xfd::SlabArgs<T>& a, const xfd::Grid& g) {
               a.extA[0] >= g.nx && a.extA[1] >= g.ny && a.extB[0] >= g.nx && a.extB[1] >= g.ny &&
               a.lo[2] == a.start && a.ext[2] == a.n,
           "z CPML slab shape");
-  require(static_cast<int64_t>(a.ext[0]) * a.ext[1] * a.ext[2] < (int64_t{1} << 30), "z CPML slab too large");
+  require(static_cast<int64_t>(a.ext[0]) * a.ext[1] * a.ext[2] < xfd::kZSlabPoints, "z CPML slab too large");
   xfd::ZSlab<T> z{};
   z.klo = a.start;
   z.khi = a.start + a.n;

@@ -110,10 +110,13 @@ __device__ __forceinline__ void cpmlFused(const CpmlList<T>& P, uint32_t mask, i
 // at use with value selects between the two uniform pointers (no
 // runtime-indexed aggregate, which would go to scratch memory, and no
 // long-lived per-lane pointers).
+// t: a point's place among the slab's pairs, 32 bits unsigned.
+constexpr int64_t kZSlabPoints = int64_t{1} << 31;  // a slab holds fewer
+static_assert(2 * (kZSlabPoints - 1) + 1 <= UINT32_MAX);
 template <class T>
 struct ZLane {
   bool in = false, sel = false;
-  int t = 0, step = 0;
+  uint32_t t = 0, step = 0;
   T ca = T(0), cb = T(0);
 };
 
@@ -134,8 +137,8 @@ __device__ __forceinline__ ZLane<T> zLane(const ZCpml<T>& Z, int i0, int j, int 
   const T* cb = in1 ? s1.cb : s0.cb;
   L.ca = ca[k - klo];
   L.cb = cb[k - klo];
-  L.step = 2 * ext1 * ext2;
-  L.t = 2 * ((i0 * ext1 + j) * ext2 + (k - klo));
+  L.step = 2u * static_cast<uint32_t>(ext1 * ext2);
+  L.t = 2u * static_cast<uint32_t>((i0 * ext1 + j) * ext2 + (k - klo));
   return L;
 }
 
