@@ -59,3 +59,15 @@ def test_line_steps_match_separate_launches(monkeypatch, nz, tfsf, faces, precis
         for x, y in zip(a.monitor_records(m), b.monitor_records(m)):
             np.testing.assert_array_equal(x, y)
     assert np.abs(b.field("EX")).max() > 0
+
+
+def test_device_bytes_count_the_lists_of_a_path(monkeypatch):
+    """What a 1D grid stepped many times per launch holds beyond separate
+    launches is counted: the addends of its TFSF corrections, 4096 steps of doubles each, and its lists."""
+    held = []
+    for env in ("0", None):
+        monkeypatch.setenv("XFD_STEP_FUSED", env) if env else monkeypatch.delenv("XFD_STEP_FUSED", raising=False)
+        sim = native.Simulation(_line(200, 12), "f64")
+        sim.init(4)
+        held.append(sim.device_bytes())
+    assert held[1] - held[0] >= 3 * 4096 * 8

@@ -346,6 +346,7 @@ struct xfd_ctx {
     for (auto& s : slabs) {
       for (auto& x : s->cpsi) b += x.bytes;
       for (auto& x : s->psi) b += x.bytes;
+      b += s->psi_h2.bytes;
       b += s->ae.bytes + s->be.bytes + s->ah.bytes + s->bh.bytes;
     }
     b += pool.bytes + rec_e.bytes + seg_e.bytes + rec_h.bytes + seg_h.bytes + state.bytes;
@@ -358,6 +359,10 @@ struct xfd_ctx {
     for (int q = 0; q < 3; ++q) b += ade_j[q].bytes + ade_jp[q].bytes + ade_eprev[q].bytes;
     for (auto& gth : gathers) b += gth->out.bytes;
     b += ckpt.bytes + far_ws.bytes;
+    for (const DevBuf* x : {&loc_e, &loc_h, &line_extra, &line_add_e, &line_add_h, &half_e, &half_h, &rec_off_e,
+                            &seg_of_e, &rec_off_h, &seg_of_h, &probe_off, &probe_of, &cpml_list_e, &cpml_list_h})
+      b += x->bytes;
+    for (auto& f : fields_b) b += f.bytes;
     b += line_terms.bytes + line_off.bytes + line_scale.bytes + line_out.bytes;
     return b;
   }
