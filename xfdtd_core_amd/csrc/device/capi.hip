@@ -291,6 +291,9 @@ struct xfd_ctx {
   bool half = false;
   // the z slabs' corrections come before the x / y slabs' (FP32 rounding only)
   bool z_first = false;
+  // what the grid and its corrections allow; a write of values that should stay
+  // zero turns half, line and te_zero off until xfd_reset
+  bool half_ok = false, line_ok = false, te_zero_ok = false;
   int half_tk = 64, half_tj = 4, half_chunk = 4;  // tile: k-lanes x j-rows x i-planes
   // the far planes i = nx, j = ny, k = nz hold zeros, which their slab
   // corrections keep (they draw on each other only), so no launch visits them
@@ -299,6 +302,7 @@ struct xfd_ctx {
   // then by work-item
   bool line = false;
   int line_threads = 0, line_extra_e = 0, line_extra_h = 0;
+  std::vector<int32_t> line_col1[2];  // cells of the column (0, 1) that it moves: Ex's, Hy's
   DevBuf loc_e, loc_h, line_extra, line_add_e, line_add_h;
   DevBuf half_e, half_h;  // HalfSlabs of each half-step
   DevBuf rec_off_e, seg_of_e, rec_off_h, seg_of_h, probe_off, probe_of;
@@ -734,7 +738,7 @@ void lineSetup(xfd_ctx& c, const std::vector<xfd::Record>& re, const std::vector
     return false;
   };
   int extra[2] = {0, 0};
-  std::vector<int32_t> loc[2], extra_cell;
+  std::vector<int32_t> loc[2], col1[2];  // H, E
   for (int is_e = 0; is_e < 2; ++is_e) {
     const auto& rec = is_e ? re : rh;
     const auto& seg = is_e ? se : sh;
@@ -742,7 +746,7 @@ void lineSetup(xfd_ctx& c, const std::vector<xfd::Record>& re, const std::vector
       const auto& r = rec[seg[q]];
       const int64_t column = r.target / c.g.pz, k = r.target % c.g.pz;
       if (r.field != (is_e ? 0 : 4) || column > 1 || (column == 1 && inReach(is_e != 0, k))) return;
-      if (is_e && column) extra_cell.push_back(static_cast<int32_t>(k));
+      if (column) col1[is_e].push_back(static_cast<int32_t>(k));
       loc[is_e].push_back(static_cast<int32_t>(column ? c.g.nz + 1 + extra[is_e]++ : k));
     }
   }
@@ -766,7 +770,9 @@ void lineSetup(xfd_ctx& c, const std::vector<xfd::Record>& re, const std::vector
   uploadVector(loc[1], c.loc_e);
   uploadVector(loc[0], c.loc_h);
   c.line_threads = static_cast<int>(std::min<int64_t>(xfd::kLineThreads, (c.g.nz + 64) / 64 * 64));
-  uploadVector(extra_cell, c.line_extra);
+  uploadVector(col1[1], c.line_extra);
+  c.line_col1[0] = col1[1];
+  c.line_col1[1] = col1[0];
   // a column's correction goes to the cell's work-item; the other column's to
   // one of the next wavefront, so the two run side by side
   const int64_t w = c.line_threads;
@@ -1443,6 +1449,9 @@ void createTyped(xfd_ctx& c, const xfd_desc& d) {
   }
   halfSetup(c, re, se, rh, sh, probes, records_meet_slabs);
   lineSetup(c, re, se, rh, sh, probes);
+  c.half_ok = c.half;
+  c.line_ok = c.line;
+  c.te_zero_ok = c.te_zero;
   if (c.half) {
     uploadVector(halfSlabs<T>(c, true), c.half_e);
     uploadVector(halfSlabs<T>(c, false), c.half_h);
@@ -1915,6 +1924,9 @@ void stepTyped(xfd_ctx& c, int64_t t0, int64_t n, bool record = true) {
 // inductor currents, ADE state, NF2FF accumulators and recordings.
 void resetState(xfd_ctx& c) {
   c.far_zero = true;
+  c.half = c.half_ok;
+  c.line = c.line_ok;
+  c.te_zero = c.te_zero_ok;
   auto zero = [&](DevBuf& b) {
     if (b.p && b.bytes) XFD_HIP(hipMemsetAsync(b.p, 0, b.bytes, c.stream));
   };
@@ -2685,14 +2697,21 @@ int xfd_read_field(xfd_ctx* c, int32_t field, double* dst) {
 int xfd_write_field(xfd_ctx* c, int32_t field, const double* src) {
   return guard([&] {
     require(c && src && field >= 0 && field < 6, "bad argument");
-    if (field == 0 || field == 1 || field == 5) c->te_zero = false;  // no longer known to stay zero
-    if (c->line && field != 5) {  // 1D: what is not Ex or Hy of the column (0, 0) no longer stays zero
-      const int64_t n = field == 0 ? c->g.nz + 1 : c->g.nz;
-      c->line = field == 0 || field == 4;
-      for (int64_t k = n; k < 2 * n && c->line; ++k) c->line = src[k] == 0.0;
-    }
     int ext[3];
     extentOf(field, c->g.nx, c->g.ny, c->g.nz, ext);
+    const int64_t values = static_cast<int64_t>(ext[0]) * ext[1] * ext[2];
+    // 2D: Ex, Ey and Hz stay zero as long as zeros are written
+    if (c->te_zero && (field == 0 || field == 1 || field == 5))
+      c->te_zero = std::all_of(src, src + values, [](double v) { return v == 0.0; });
+    // 1D: so does what is not Hz, or Ex or Hy of the column (0, 0) and the points
+    // of (0, 1) that a correction moves
+    if (c->line && field != 5) {
+      const bool moves = field == 0 || field == 4;
+      const int64_t n = field == 0 ? c->g.nz + 1 : c->g.nz;
+      const auto& col1 = c->line_col1[field == 0 ? 0 : 1];
+      for (int64_t q = moves ? n : 0; q < values && c->line; ++q)
+        c->line = src[q] == 0.0 || (moves && q < 2 * n && std::find(col1.begin(), col1.end(), q - n) != col1.end());
+    }
     if (c->half && c->far_zero) {  // a far plane that no longer holds zeros takes its slab corrections
       const int n[3] = {c->g.nx, c->g.ny, c->g.nz};
       bool zero = true;
@@ -2988,7 +3007,7 @@ int xfd_batch_create(int32_t n, const xfd_desc* descs, xfd_batch** out) {
       // one launch took 203 us where sweep, slabs and records take 210 (16 cases
       // of 48..128 cells a side, FP32), and the sweeps with only the z slabs
       // inside were slower.
-      c->half = false;
+      c->half = c->half_ok = false;
       c->zfused = false;
       std::fill(c->zslab.begin(), c->zslab.end(), 0);
       b->shared = b->shared && c->classed && !c->wide && c->tdnfs.empty();
