@@ -481,7 +481,6 @@ xfd::CoefPtrs<T> coefPtrs(xfd_ctx& c) {
   return C;
 }
 
-// Uploads a double array of the reference extent into a padded device array.
 void checkHip(hipError_t e) { XFD_HIP(e); }
 
 // `count` doubles of device memory to the host.
@@ -496,6 +495,7 @@ void readDoubles(xfd_ctx& c, const double* src, double* dst, size_t count) {
       });
 }
 
+// Uploads a double array of the reference extent into a padded device array.
 template <class T>
 void uploadPadded(xfd_ctx& c, const double* host, const int ext[3], T* dst, DevBuf& staging) {
   const size_t n = static_cast<size_t>(ext[0]) * ext[1] * ext[2];

@@ -5,6 +5,8 @@
 
 #include <algorithm>
 #include <cstdlib>
+#include <stdexcept>
+#include <string>
 
 #include "adjoint_kernels.hpp"
 #include "batch_kernels.hpp"
@@ -594,9 +596,10 @@ void launchLine(hipStream_t s, const Coef& K, const LineArgs<T>& a, int64_t t0, 
   const size_t lds = LineLaunch<T>::ldsBytes(a.nz, a.extra_e + a.extra_h,
                                              (a.slabs > 0 ? a.e[0].n : 0) + (a.slabs > 1 ? a.e[1].n : 0),
                                              a.re.held + a.rh.held);
-  if (lds > (size_t(64) << 10))  // the default limit of dynamic LDS
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_line<T, Coef, C>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+  if (lds > (size_t(64) << 10) &&  // the default limit of dynamic LDS
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&k_line<T, Coef, C>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)) != hipSuccess)
+    throw std::runtime_error("1D step: the device refuses " + std::to_string(lds) + " bytes of LDS");
   for (const auto* e : {&a.re, &a.rh})
     if (e->addends)
       hipLaunchKernelGGL(k_line_addends<T>, dim3(blocks_for(n, 256), static_cast<unsigned>(e->nseg)), dim3(256), 0, s,
