@@ -1006,3 +1006,32 @@ def test_staged_recordings(monkeypatch):
             ref.run(steps)
             for x, y in zip(a[0], ref.monitor_records(0)):
                 np.testing.assert_array_equal(x, y)
+
+
+@pytest.mark.parametrize("dim", [3, 1])
+def test_lumped_elements_at_the_far_planes_fp64(dim):
+    """Elements that reach a box's last nodes, and elements on a line, whose
+    cross section is one cell: the nodes on a far plane take no correction."""
+    dl, inf = 1e-3, float("inf")
+    wave = S.Waveform.gaussian(10e-12, 20e-12)
+    s = S.Simulation(dl, dl, dl, 0.9)
+    n = [12 * dl, 10 * dl, 20 * dl]
+    lo, size = (S.Vector(0, 0, 0), S.Vector(*n)) if dim == 3 else (S.Vector(-inf, -inf, 0), S.Vector(inf, inf, n[2]))
+    s.addObject(S.Object("domain", S.Cube(lo, size), S.Material.createAir()))
+
+    def box(i, j, k, di, dj, dk):
+        if dim == 1:
+            return S.Cube(S.Vector(-inf, -inf, k * dl), S.Vector(inf, inf, dk * dl))
+        return S.Cube(S.Vector(i * dl, j * dl, k * dl), S.Vector(di * dl, dj * dl, dk * dl))
+
+    s.addObject(S.CurrentSource("i", box(4, 7, 9, 2, 3, 2), "XP", 2.0, wave))     # to the far y plane
+    s.addObject(S.VoltageSource("v", box(4, 2, 15, 2, 2, 5), "XP", 50.0, wave))   # to the far z plane
+    s.addObject(S.Inductor("l", box(4, 4, 5, 2, 6, 1), "X", 1e-9))
+    s.addObject(S.Resistor("r", box(4, 8, 12, 2, 2, 1), "X", 75.0))
+    sp, steps = s.spec(), 80
+    ref, dev = RefSim(sp), native.Simulation(sp, "f64")
+    ref.run(steps)
+    dev.run(steps)
+    for f in FIELDS:
+        np.testing.assert_array_equal(dev.field(f), ref.field(f), err_msg=f)
+    assert np.abs(ref.field("EX")).max() > 0

@@ -993,6 +993,17 @@ struct Simulation::Impl {
       lo[a] = o[a];
       cnt[a] = a == m ? e[a] - o[a] : e[a] - o[a] + 1;
     }
+    // The corrector's task is the element's cells cut to [0, N)
+    // (lumped_element.cpp:154-158, inductor.cpp:111-135): nodes on a far plane
+    // are patched but not corrected.  A one-cell axis (1D, 2D) has no size there,
+    // and its far nodes are never updated: they are left alone.
+    std::size_t run[3], vol = 1;
+    for (int a = 0; a < 3; ++a) {
+      const std::size_t sizes = a == m ? e_size[a].size() : h_size[a].size();
+      cnt[a] = std::min(cnt[a], sizes - std::min(sizes, lo[a]));
+      run[a] = std::min(cnt[a], N[a] - std::min<std::size_t>(N[a], lo[a]));
+      vol *= run[a];
+    }
     const Real gmain = static_cast<Real>(e[m] - o[m]);
     const std::size_t ga = e[A] - o[A] + 1, gb = e[B] - o[B] + 1;
     const std::size_t gc = e[m] - o[m];
@@ -1025,15 +1036,14 @@ struct Simulation::Impl {
       // (L' da db), cecjc = -2 dt / (2 eps + dt sigma); no coefficient patch
       const Real lf = ind->inductance() * ga * gb / gc;
       LumpedData ld;
-      const std::size_t vol = cnt[0] * cnt[1] * cnt[2];
       ld.coff.resize(vol);
       ld.coff_j.resize(vol);
-      for (std::size_t i = 0; i < cnt[0]; ++i)
-        for (std::size_t j = 0; j < cnt[1]; ++j)
-          for (std::size_t k = 0; k < cnt[2]; ++k) {
+      for (std::size_t i = 0; i < run[0]; ++i)
+        for (std::size_t j = 0; j < run[1]; ++j)
+          for (std::size_t k = 0; k < run[2]; ++k) {
             const std::size_t g[3] = {lo[0] + i, lo[1] + j, lo[2] + k};
             const Real da = size_of(A, g[A]), db = size_of(B, g[B]), dc = size_of(m, g[m]);
-            const std::size_t q = (i * cnt[1] + j) * cnt[2] + k;
+            const std::size_t q = (i * run[1] + j) * run[2] + k;
             ld.coff_j[q] = dt * dc / (lf * da * db);
             ld.coff[q] = -(2 * dt) / (2 * eps[m].at(g[0], g[1], g[2]) + dt * se[m].at(g[0], g[1], g[2]));
           }
@@ -1041,9 +1051,9 @@ struct Simulation::Impl {
       ld.d.component = m;
       for (int a = 0; a < 3; ++a) {
         ld.d.origin[a] = static_cast<int32_t>(lo[a]);
-        ld.d.size[a] = static_cast<int32_t>(cnt[a]);
+        ld.d.size[a] = static_cast<int32_t>(run[a]);
       }
-      lumped.push_back(std::move(ld));
+      if (vol) lumped.push_back(std::move(ld));
       return;
     }
     auto* res = dynamic_cast<Resistor*>(&le);
@@ -1063,7 +1073,7 @@ struct Simulation::Impl {
     const Field3& ep = eps[m];
     const Field3& sg = se[m];
     LumpedData ld;
-    ld.coff.resize(cnt[0] * cnt[1] * cnt[2]);
+    ld.coff.resize(vol);
     for (std::size_t i = 0; i < cnt[0]; ++i)
       for (std::size_t j = 0; j < cnt[1]; ++j)
         for (std::size_t k = 0; k < cnt[2]; ++k) {
@@ -1080,19 +1090,21 @@ struct Simulation::Impl {
           cece.at(g[0], g[1], g[2]) = (2 * e0 - dt * s0 - beta) / (2 * e0 + dt * s0 + beta);
           cecha.at(g[0], g[1], g[2]) = -2 * dt / ((2 * e0 + dt * s0 + beta) * db);
           cechb.at(g[0], g[1], g[2]) = 2 * dt / ((2 * e0 + dt * s0 + beta) * da);
-          const std::size_t q = (i * cnt[1] + j) * cnt[2] + k;
+          if (i >= run[0] || j >= run[1] || k >= run[2]) continue;
+          const std::size_t q = (i * run[1] + j) * run[2] + k;
           if (vs) ld.coff[q] = -2 * dt / ((2 * e0 + dt * s0 + beta) * alpha) * factor;
           if (cs) ld.coff[q] = -2 * dt / ((2 * e0 + dt * s0 + beta) * (db * da)) * factor;
         }
     if (res) return;
+    Waveform& w = vs ? vs->waveform() : cs->waveform();
+    w.init(hTime());  // voltage_source.cpp:163-167
+    if (!vol) return;
+    ld.wave = w.value();
     ld.d.component = m;
     for (int a = 0; a < 3; ++a) {
       ld.d.origin[a] = static_cast<int32_t>(lo[a]);
-      ld.d.size[a] = static_cast<int32_t>(cnt[a]);
+      ld.d.size[a] = static_cast<int32_t>(run[a]);
     }
-    Waveform& w = vs ? vs->waveform() : cs->waveform();
-    w.init(hTime());  // voltage_source.cpp:163-167
-    ld.wave = w.value();
     lumped.push_back(std::move(ld));
   }
 
