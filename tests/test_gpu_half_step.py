@@ -8,6 +8,7 @@ import ctypes
 import numpy as np
 import pytest
 
+from oracle import RefSim
 from xfdtd_core_amd import native
 from xfdtd_core_amd import spec as S
 
@@ -220,3 +221,81 @@ def test_fp32_keeps_the_field_product_unrounded(monkeypatch, on):
     unit = np.spacing(np.maximum(np.abs(got), np.abs(want)).astype(np.float32))
     assert (np.abs(got - want) <= 0.5 * unit + 2.0**-24 * np.abs(ad)).all()
     assert np.abs(got - e[:, 1:-1, 1:-1]).max() > 0
+
+
+def _poles(kind, n):
+    """A material of n poles; the modified Lorentz scheme also where kinds mix."""
+    w = [2e10 * (1 + 0.7 * p) for p in range(n)]
+    if kind == "drude":
+        return S.DrudeMedium.makeDrudeMedium("d", 2.0, [0.6 * v for v in w], [1e9 * (1 + p) for p in range(n)])
+    if kind == "debye":
+        return S.DebyeMedium.makeDebyeMedium("d", 2.0, [3.0 + p for p in range(n)], [1e-11 * (1 + p) for p in range(n)])
+    return S.LorentzMedium.makeMLorentz("d", 2.0, [0.4 * v * v for v in w], [2e9] * n, [v * v for v in w],
+                                        [2e9 * (1 + p) for p in range(n)], [1.0] * n)
+
+
+# room for two poles, for four, and the loop over more
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("kind", ["drude", "debye", "lorentz"])
+def test_dispersive_half_step(monkeypatch, kind, n):
+    """A dispersive block in a driven box: FP64 the oracle's bits, and in both
+    precisions those of a launch per correction."""
+    dl, pml, inner, steps = 1e-3, 5, (14, 13, 60), 60
+    s = S.Simulation(dl, dl, dl, 0.9)
+    s.addObject(S.Object("domain", S.Cube(S.Vector(0, 0, 0), S.Vector(*[m * dl for m in inner])),
+                         S.Material.createAir()))
+    s.addObject(S.Object("block", S.Cube(S.Vector(0, 4 * dl, 10 * dl), S.Vector(14 * dl, 5 * dl, 30 * dl)),
+                         _poles(kind, n)))
+    s.addObject(S.CurrentSource("i", S.Cube(S.Vector(7 * dl, 2 * dl, 9 * dl), S.Vector(0, 0, dl)), "ZP", 1e3,
+                                S.Waveform.gaussian(10e-12, 20e-12)))
+    for f in ("XN", "XP", "YN", "YP", "ZN", "ZP"):
+        s.addBoundary(S.PML(pml, f))
+    spec = s.spec()
+    ref = RefSim(spec)
+    ref.run(steps)
+    for precision in ("f64", "f32"):
+        a = _run(monkeypatch, spec, precision, steps, True)
+        b = _run(monkeypatch, spec, precision, steps, False)
+        for sim in (a, b):
+            sim.advance(0, steps)
+            sim.finish()
+        _compare(a, b, precision, f"{kind} {n}")
+        if precision == "f64":
+            for f in FIELDS:
+                np.testing.assert_array_equal(a.field(f), ref.field(f), err_msg=f)
+
+
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+@pytest.mark.parametrize("layout", ["classed", "wide", "dense"])
+def test_half_step_coefficient_layouts(monkeypatch, layout, precision):
+    """16-bit class ids, 32-bit ones (80000 distinct triples a component) and
+    dense coefficients: the bits of a launch per correction."""
+    n, rng = (70, 66, 75), np.random.default_rng(2)
+    monkeypatch.setenv("XFD_COEF_MODE", "dense" if layout == "dense" else "")
+    classes = 80000 if layout == "wide" else 50
+    coeffs = {}
+    for name in native.COEFF_NAMES:
+        c, e = "xyz".index(name[2]), name[1] == "e"
+        ext = tuple(m + (1 if (q == c) != e else 0) for q, m in enumerate(n))
+        if len(name) == 4:  # the component's own coefficient comes first
+            ids = rng.integers(0, classes, ext)
+        lo, hi = (0.7, 1.0) if len(name) == 4 else (-0.3, 0.3)
+        coeffs[name] = rng.uniform(lo, hi, classes)[ids]
+    start = None
+    out = []
+    for on in (True, False):
+        monkeypatch.setenv("XFD_CPML_INSWEEP", "1" if on else "0")
+        ctx = native.Context(coeffs, precision)
+        mode = ctypes.c_int32()
+        assert native.load_library().xfd_cpml_fused(ctx._h, ctypes.byref(mode)) == 0 and mode.value == (4 if on else 0)
+        assert ctx.coef_layout()[0] == (layout != "dense")
+        assert (max(ctx.coef_layout()[1]) > 65535) == (layout == "wide")
+        start = start or {f: rng.standard_normal(ctx.extent(f)) for f in FIELDS}
+        for f in FIELDS:
+            ctx.write(f, start[f])
+        ctx.step(0, 6)
+        out.append({f: ctx.read(f) for f in FIELDS})
+        ctx.close()
+    for f in FIELDS:
+        np.testing.assert_array_equal(out[0][f], out[1][f], err_msg=f)
+        assert np.isfinite(out[0][f]).all()
