@@ -38,10 +38,12 @@ def test_read_returns_what_was_written(n, dtype):
     assert room[0] == room[-1] == room[-2] == -1.0
 
 
-def test_reads_from_several_threads():
-    n = (90, 80, 70)
+# four reads run at a time; more wait, and small reads do beside large ones
+@pytest.mark.parametrize("sizes", [[(90, 80, 70)] * 3, [(90, 80, 70), (5, 6, 7), (64, 64, 64)] * 3,
+                                   [(150, 140, 130)] * 2 + [(9, 9, 9)] * 6])
+def test_reads_from_several_threads(sizes):
     jobs = []
-    for q in range(3):
+    for q, n in enumerate(sizes):
         ctx = _context(n, "f64")
         v = np.random.default_rng(q).standard_normal((n[0], n[1] + 1, n[2] + 1))
         ctx.write("EX", v)

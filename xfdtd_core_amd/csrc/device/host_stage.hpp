@@ -7,8 +7,16 @@
 // way, so half the bytes cross the bus.  Measured, six 384^3 FP32 fields (1.4 GB
 // to 2.7 GB): 165 -> 31 ms.
 //
-// The slots are shared by every context of the process, one read at a time, and
-// freed with the last context.
+// The slots are shared by every context of the process: up to kSets reads at a
+// time, each with slots of its own, made for the first read that finds none free,
+// grown to the largest read (at most 32 MB) and freed with the last context.
+// Reads of several contexts at once, us each over all of 1 / 4 / 8 threads, FP64:
+// pageable copies 64^3 215 / 125 / 105, 100^3 560 / 310 / 280; one read at a time
+// with eight host threads 164 / 145 / 154 and 376 / 365 / 381; four with eight 165 /
+// 115 / 117 and 375 / 288 / 283; four with four, as here, 152 / 97 / 90 and 320 / 203
+// / 183.  Two host threads are faster still into memory in use (64^3 135 / 65 / 57)
+// but not into fresh memory, whose pages they touch first (300^3 FP32 50 ms against
+// 30; pageable 59).
 #pragma once
 
 #include <emmintrin.h>
@@ -16,6 +24,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <condition_variable>
 #include <cstdint>
 #include <cstring>
 #include <exception>
@@ -30,20 +39,19 @@ class HostStage {
   static constexpr size_t kSlotBytes = size_t(2) << 20;
   static constexpr size_t kSlots = 16;
   static constexpr size_t kMinItems = size_t(64) << 10;  // per chunk, where a read is split
-  static constexpr size_t kThreads = 8;
+  static constexpr size_t kThreads = 4;
+  static constexpr size_t kSets = 4;
 
   // One per context: the slots live while any does.
   struct User {
     User() {
-      std::lock_guard<std::mutex> lock(mu());
-      ++users();
+      std::lock_guard<std::mutex> lock(pool().mu);
+      ++pool().users;
     }
     ~User() {
-      std::lock_guard<std::mutex> lock(mu());
-      if (--users() == 0 && base()) {
-        (void)hipHostFree(base());
-        base() = nullptr;
-      }
+      std::lock_guard<std::mutex> lock(pool().mu);
+      if (--pool().users > 0) return;
+      for (Set& set : pool().sets) set.release();
     }
     User(const User&) = delete;
     User& operator=(const User&) = delete;
@@ -55,17 +63,13 @@ class HostStage {
   template <class Check, class Enqueue, class Take>
   static void read(hipStream_t stream, size_t items, size_t item, Check check, Enqueue enqueue, Take take) {
     if (items == 0) return;
-    check(hipStreamSynchronize(stream));  // what came before, without holding the slots
-    std::lock_guard<std::mutex> lock(mu());
-    if (!base()) {
-      void* p = nullptr;
-      check(hipHostMalloc(&p, kSlotBytes * kSlots, hipHostMallocPortable));
-      base() = static_cast<unsigned char*>(p);
-    }
+    check(hipStreamSynchronize(stream));  // what came before, without holding slots
     const size_t most = kSlotBytes / item;
     const size_t per = std::min(most, std::max(kMinItems, (items + kSlots - 1) / kSlots));
     const size_t chunks = (items + per - 1) / per;
-    auto slot = [&](size_t c) { return base() + (c % kSlots) * kSlotBytes; };
+    const size_t pitch = (per * item + 255) / 256 * 256;
+    const Lease slots(std::min(chunks, kSlots) * pitch, check);
+    auto slot = [&](size_t c) { return slots.base() + (c % kSlots) * pitch; };
     auto count = [&](size_t c) { return std::min(per, items - c * per); };
     if (chunks == 1) {
       enqueue(size_t(0), items, slot(0));
@@ -139,18 +143,77 @@ class HostStage {
  private:
   static __m128d pairAt(const double* p) { return _mm_loadu_pd(p); }
   static __m128d pairAt(const float* p) { return _mm_set_pd(static_cast<double>(p[1]), static_cast<double>(p[0])); }
-  static std::mutex& mu() {
-    static std::mutex m;
-    return m;
-  }
-  static int& users() {
-    static int n = 0;
-    return n;
-  }
-  static unsigned char*& base() {
-    static unsigned char* p = nullptr;
+  // The slots of one read.
+  struct Set {
+    unsigned char* p = nullptr;
+    size_t bytes = 0;
+    bool busy = false;
+    void release() {
+      if (p) (void)hipHostFree(p);
+      p = nullptr;
+      bytes = 0;
+    }
+  };
+  struct Pool {
+    std::mutex mu;
+    std::condition_variable freed;
+    int users = 0;
+    Set sets[kSets];
+  };
+  static Pool& pool() {
+    static Pool& p = *new Pool;  // outlives contexts that live until the process ends
     return p;
   }
+
+  // A set for the time of a read: a free one that is large enough, else the
+  // largest free one, grown, so that reads one after the other share a set.
+  class Lease {
+   public:
+    template <class Check>
+    Lease(size_t need, Check check) {
+      size_t bytes = size_t(64) << 10;
+      while (bytes < need) bytes *= 2;
+      Pool& P = pool();
+      {
+        std::unique_lock<std::mutex> lock(P.mu);
+        auto pick = [&]() -> Set* {
+          Set* best = nullptr;
+          for (Set& s : P.sets)
+            if (!s.busy && (!best || (best->bytes < bytes ? s.bytes > best->bytes
+                                                          : s.bytes >= bytes && s.bytes < best->bytes)))
+              best = &s;
+          return best;
+        };
+        P.freed.wait(lock, [&] { return (set_ = pick()) != nullptr; });
+        set_->busy = true;
+      }
+      if (set_->bytes >= bytes) return;
+      try {
+        set_->release();
+        void* p = nullptr;
+        check(hipHostMalloc(&p, bytes, hipHostMallocPortable));
+        set_->p = static_cast<unsigned char*>(p);
+        set_->bytes = bytes;
+      } catch (...) {
+        giveBack();
+        throw;
+      }
+    }
+    ~Lease() { giveBack(); }
+    Lease(const Lease&) = delete;
+    Lease& operator=(const Lease&) = delete;
+    unsigned char* base() const { return set_->p; }
+
+   private:
+    void giveBack() {
+      {
+        std::lock_guard<std::mutex> lock(pool().mu);
+        set_->busy = false;
+      }
+      pool().freed.notify_one();
+    }
+    Set* set_ = nullptr;
+  };
 };
 
 }  // namespace xfd
