@@ -239,7 +239,8 @@ def _poles(kind, n):
 @pytest.mark.parametrize("kind", ["drude", "debye", "lorentz"])
 def test_dispersive_half_step(monkeypatch, kind, n):
     """A dispersive block in a driven box: FP64 the oracle's bits, and in both
-    precisions those of a launch per correction."""
+    precisions those of a launch per correction, of all of them or of the E
+    half-step's alone (the arrangement of large grids)."""
     dl, pml, inner, steps = 1e-3, 5, (14, 13, 60), 60
     s = S.Simulation(dl, dl, dl, 0.9)
     s.addObject(S.Object("domain", S.Cube(S.Vector(0, 0, 0), S.Vector(*[m * dl for m in inner])),
@@ -260,9 +261,30 @@ def test_dispersive_half_step(monkeypatch, kind, n):
             sim.advance(0, steps)
             sim.finish()
         _compare(a, b, precision, f"{kind} {n}")
+        with monkeypatch.context() as m:
+            m.setenv("XFD_ADE_E", "apart")
+            e = _run(m, spec, precision, steps, True)
+            e.set_profiling(True)
+            e.advance(0, steps)
+            e.finish()
+            launches = {k: v[0] for k, v in e.kernel_stats().items()}
+            assert launches.get("cpml_h", 0) == 0 and launches["cpml_e"] > 0
+        _compare(e, b, precision, f"{kind} {n} E apart")
         if precision == "f64":
             for f in FIELDS:
                 np.testing.assert_array_equal(a.field(f), ref.field(f), err_msg=f)
+
+
+# where the one launch loses: FP32 rows of whole 128-lane tiles past 128 MiB
+@pytest.mark.parametrize("n,mode", [((130, 130, 256), 0), ((130, 130, 250), 4), ((64, 64, 128), 4)])
+def test_large_dispersive_grids_keep_separate_launches(n, mode):
+    dl = 1e-3
+    s = S.Simulation(dl, dl, dl, 0.9)
+    s.addObject(S.Object("domain", S.Cube(S.Vector(0, 0, 0), S.Vector(*[m * dl for m in n])), S.Material.createAir()))
+    s.addObject(S.Object("block", S.Cube(S.Vector(0, 0, 0), S.Vector(9 * dl, 9 * dl, 9 * dl)), _poles("debye", 1)))
+    sim = native.Simulation(s.spec(), "f32")
+    sim.init(1)
+    assert sim.cpml_fused() == mode
 
 
 @pytest.mark.parametrize("precision", ["f64", "f32"])

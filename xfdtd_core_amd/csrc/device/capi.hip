@@ -289,6 +289,7 @@ struct xfd_ctx {
   // each half-step (update, every CPML slab, records, point probes) as one
   // launch (k_half), with its records and probes by tile
   bool half = false;
+  bool half_h_only = false;  // dispersive: the E half-step as a launch per correction
   // the z slabs' corrections come before the x / y slabs' (FP32 rounding only)
   bool z_first = false;
   // what the grid and its corrections allow; a write of values that should stay
@@ -809,6 +810,31 @@ void halfSetup(xfd_ctx& c, const std::vector<xfd::Record>& re, const std::vector
            !is("XFD_CPML_INSWEEP", '0') && !is("XFD_STEP_FUSED", '0') && !is("XFD_CPML_FUSED", '1') &&
            !is("XFD_CPML_ZFUSED", '1');
   if (!c.half) return;
+  // The dispersive E half-step holds two waves fewer per SIMD than the update and
+  // the slabs apart, which large grids feel, most on rows of whole 128-lane tiles
+  // (the update's own tile; k_half is faster on 64 x 4 there).  Small ones are
+  // bound by the launches.  us a step, one launch each / H alone / neither, for
+  // slabs of three materials in half of the box; two-pole Lorentz in a sixth:
+  //   FP32 128^3 126 / 142 / 148; 99 / 123 / 132   160^3 212 / 205 / 211; 169 / 165 / 178
+  //        192^3 354 / 340 / 354; 269 / 262 / 276  240^3 697 / 671 / 677; 593 / 602 / 606
+  //        160 x 160 x 128 186 / 181 / 181; 171 / 160 / 164
+  //        256^3 855 / 765 / 752; 690 / 629 / 614  384^3 2383 / 2273 / 2254
+  //   FP64 128^3 219 / 228 / 230; 192 / 195 / 209  192^3 598 / 611 / 630; 437 / 447 / 464
+  //        160 x 160 x 128 317 / 328 / 339; 289 / 265 / 270
+  //        256^3 1421 / 1378 / 1370; 1229 / 1093 / 1085  320^3 2263 / 2328 / 2379; 1666 / 1679 / 1720
+  // How the materials lie among the tiles decides by up to 6 % past 200^3 in FP64
+  // (224^3: 928 / 973 / 983 and 944 / 912 / 920); H alone is never the slowest.
+  if (c.ade_scheme >= 0) {
+    const int64_t mib = g.total * (6 * c.elem + 12) >> 20;  // a step's fields and class ids
+    const bool rows128 = g.nz % 128 == 0;
+    c.half_h_only = mib > (rows128 ? 192 : c.elem == 4 ? 256 : 512);
+    c.half = !(c.elem == 4 && rows128 && mib > 128);
+    if (const char* e = std::getenv("XFD_ADE_E")) {  // "half", "apart": one launch, or one per correction
+      c.half = true;
+      c.half_h_only = e[0] == 'a';
+    }
+    if (!c.half) return;
+  }
   // FP32 rows on which the sweeps would take the z slabs (zfused) keep the order
   // that has: results do not depend on which of the two paths a grid takes.
   c.z_first = c.zfused;
@@ -816,7 +842,12 @@ void halfSetup(xfd_ctx& c, const std::vector<xfd::Record>& re, const std::vector
   c.n_fused = 0;
   c.zfused = false;
   std::fill(c.zslab.begin(), c.zslab.end(), 0);
-  if (c.dim == 3 && xfd::sweepTile128(g)) {
+  // tile as the sweeps' (us a step, 64 x 4 / 128 x 2: 384^3 FP32 1066 / 1049, FP64
+  // 2076 / 2026; 256^3 FP32 382 / 344, FP64 713 / 663; 128^3 FP32 59.8 / 59.2, FP64
+  // 84.2 / 85.4); the dispersive E half-step stays on 64 x 4 (128^3 FP32 120 / 131, FP64
+  // 221 / 234)
+  if (c.dim == 3 && xfd::sweepTile128(g) &&
+      (c.ade_scheme < 0 || c.half_h_only || std::getenv("XFD_SWEEP_TILE"))) {
     c.half_tk = 128;
     c.half_tj = 2;
   }
@@ -830,7 +861,12 @@ void halfSetup(xfd_ctx& c, const std::vector<xfd::Record>& re, const std::vector
   }
   int64_t nbx = (g.nz + c.half_tk - 1) / c.half_tk, nby = (g.ny + c.half_tj - 1) / c.half_tj;
   int64_t tiles = nbx * nby * ((g.nx + c.half_chunk - 1) / c.half_chunk);
-  if (c.dim == 2) {  // 64 points of a row per wavefront, a march of rows each
+  // 2D: 64 points of a row per wavefront, a march of rows each: up to 4 while
+  // 8192 wavefronts remain (us a step with 1 / 2 / 4 / 8: 330 x 350 FP64 10.3 / 11.5
+  // / 13.7 / 19.8; 1000 x 900 FP32 18.3 / 16.1 / 16.7 / 22.2; 2001 x 1501 FP32 42.9 /
+  // 35.8 / 33.3 / 32.1, FP64 52.2 / 48.1 / 49.8 / 48.9; 4096^2 FP32 199 / 164 / 151 /
+  // 149)
+  if (c.dim == 2) {
     nbx = (g.ny + 63) / 64;
     if (!std::getenv("XFD_ICHUNK"))
       c.half_chunk = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(4, g.nx * nbx / 8192)));
@@ -1713,6 +1749,7 @@ void stepTyped(xfd_ctx& c, int64_t t0, int64_t n, bool record = true) {
   // the one-launch half-steps; a probe may lie on a far plane, whose
   // corrections (if any) follow the launch, so it is then sampled after them
   const bool half_probes = record && c.far_zero;
+  const bool half_e = c.half && !c.half_h_only;
   xfd::HalfArgs<T> HH{}, HE{};
   if (c.half) {
     HH = halfArgs<T>(c, false, false);
@@ -1813,11 +1850,11 @@ void stepTyped(xfd_ctx& c, int64_t t0, int64_t n, bool record = true) {
       });
       c.parity ^= 1;
       F = FB;
-    } else if (c.half) {
-      half(false, t);
-      half(true, t);
     } else {
-    c.timed(K_UPDATE_H, [&] {
+    if (c.half)
+      half(false, t);
+    else
+      c.timed(K_UPDATE_H, [&] {
       if (c.dim != 3) {
         if (c.classed)
           xfd::Launch<T>::update_low(st, c.g, F, K, c.dim, true, c.te_zero);
@@ -1831,12 +1868,12 @@ void stepTyped(xfd_ctx& c, int64_t t0, int64_t n, bool record = true) {
         xfd::Launch<T>::update_h(st, c.g, F, C, c.ichunk, PH, ZH);
       }
     });
-    if (c.nseg_h)
+    if (c.nseg_h && !c.half)
       c.timed(K_REC_H, [&] {
         xfd::Launch<T>::records(st, F, c.rec_h.as<xfd::Record>(), c.seg_h.as<int64_t>(), c.nseg_h,
                                 c.pool.as<double>(), c.state.as<T>(), t);
       });
-    for (size_t q = 0; q < sh.size(); ++q)
+    for (size_t q = 0; q < sh.size() && !c.half; ++q)
       c.timed(K_CPML_H, [&] {
         if (pairs(sh, q)) {
           xfd::Launch<T>::cpml2(st, c.g, F, sh[q], sh[q + 1], false);
@@ -1848,7 +1885,10 @@ void stepTyped(xfd_ctx& c, int64_t t0, int64_t n, bool record = true) {
         else
           xfd::Launch<T>::cpml(st, c.g, F, sh[q], false);
       });
-    c.timed(K_UPDATE_E, [&] {
+    if (half_e)
+      half(true, t);
+    else
+      c.timed(K_UPDATE_E, [&] {
       if (c.dim != 3) {
         if (c.classed)
           xfd::Launch<T>::update_low(st, c.g, F, K, c.dim, false);
@@ -1870,12 +1910,12 @@ void stepTyped(xfd_ctx& c, int64_t t0, int64_t n, bool record = true) {
       }
     });
     }
-    if (c.nseg_e && !c.half)
+    if (c.nseg_e && !half_e)
       c.timed(K_REC_E, [&] {
         xfd::Launch<T>::records(st, F, c.rec_e.as<xfd::Record>(), c.seg_e.as<int64_t>(), c.nseg_e,
                                 c.pool.as<double>(), c.state.as<T>(), t);
       });
-    for (size_t q = 0; q < se.size() && !c.fstep && !c.half; ++q)
+    for (size_t q = 0; q < se.size() && !c.fstep && !half_e; ++q)
       c.timed(K_CPML_E, [&] {
         if (pairs(se, q)) {
           xfd::Launch<T>::cpml2(st, c.g, F, se[q], se[q + 1], true);
@@ -1891,7 +1931,7 @@ void stepTyped(xfd_ctx& c, int64_t t0, int64_t n, bool record = true) {
       XFD_HIP(hipGetLastError());
       continue;
     }
-    if (c.nprobe && t < c.probe_count && !(c.half && half_probes))
+    if (c.nprobe && t < c.probe_count && !(half_e && half_probes))
       c.timed(K_GATHER, [&] {
         xfd::Launch<T>::probes(st, F, c.probe_list.as<xfd::Probe>(), c.nprobe, c.probe_out.as<double>(),
                                c.probe_count, t);
