@@ -968,7 +968,7 @@ __global__ __launch_bounds__(256) void k_far_reduce(int na, int chunks, const do
 template <class T>
 __device__ __forceinline__ double recordAdd(double a, double b, double c) {
 #pragma clang fp contract(off)
-  return sizeof(T) == sizeof(float) ? __builtin_fma(a, b, c) : a * b + c;
+  return sizeof(T) == sizeof(float) ? __builtin_fma(a, b, c) : c + a * b;
 }
 
 // A TFSF record's incident value in table row `row`: TFSFCorrector::exInc..hzInc
@@ -976,7 +976,10 @@ __device__ __forceinline__ double recordAdd(double a, double b, double c) {
 template <class T>
 __device__ __forceinline__ double recordInc(const Record& R, const double* row) {
 #pragma clang fp contract(off)
-  return R.tr * recordAdd<T>(R.omw, row[0], R.w * row[1]);
+  if constexpr (sizeof(T) == sizeof(float))
+    return R.tr * __builtin_fma(R.omw, row[0], R.w * row[1]);
+  else
+    return R.tr * (R.omw * row[0] + R.w * row[1]);
 }
 
 template <class T>
