@@ -51,7 +51,8 @@ def alg_bytes_per_launch(kernel: str, n: int, pml: int, s: int, fused: int = 0,
     separate sweep adds are actual, not algorithmic, traffic); CPML = 12 * s
     per slab cell and step (4 components x psi read + write + c_psi read), so
     one slab launch (2 components) owns 6 * s per slab cell.  Slabs applied
-    inside the sweeps (`fused` 1: the four x/y slabs, 2: the two z slabs)
+    inside the sweeps (`fused` 1: the four x/y slabs, 2: the two z slabs, 4: all
+    six, in the one-launch half-steps)
     move their share to the sweep; their separate launches only finish the
     far grid planes (not counted), and the CPML figure is the mean over the
     `cpml_launches` launches of a half-step (six, one per slab; fewer where
@@ -71,13 +72,16 @@ def alg_bytes_per_launch(kernel: str, n: int, pml: int, s: int, fused: int = 0,
 TRAFFIC_FILE = ROOT / "profiles" / "hbm_traffic_inhomogeneous_box_384.json"
 
 
-def measured_traffic(precision, n, pml):
-    """HBM bytes per launch of each kernel, from the calibrated rocprofv3
+def measured_traffic(precision, n, pml, fused):
+    """HBM bytes per launch of each kernel class, from the calibrated rocprofv3
     FETCH_SIZE / WRITE_SIZE runs recorded for the 384^3 box (None for other
-    sizes, which were not profiled)."""
+    sizes, which were not profiled, and where the step runs other kernels than
+    the profiled one: another cpml_fused())."""
     if n != 384 or pml != 12 or not TRAFFIC_FILE.exists():
         return None
     d = json.loads(TRAFFIC_FILE.read_text())
+    if d["cpml_fused"].get(precision) != int(fused):
+        return None
     return {k: v["hbm_bytes"] for k, v in d["kernels"].get(precision, {}).items()}
 
 
@@ -134,7 +138,7 @@ def run_device(sim, precision, warmup, steps, n, pml):
     kernels[dom]["timed_region"] = {"launches": dl, "avg_ms": round(dom_avg, 5)}
     ach = round(alg_bytes_per_launch(dom, n, pml, s, fused, kernels[dom]["launches"] / BREAKDOWN_STEPS)
                 / (dom_avg * 1e-3) / 1e9, 1)
-    traffic = measured_traffic(precision, n, pml)
+    traffic = measured_traffic(precision, n, pml, fused)
     for name, k in kernels.items():
         if traffic and name in traffic:
             k["hbm_bytes_pmc"] = traffic[name]
@@ -164,8 +168,10 @@ def run_device(sim, precision, warmup, steps, n, pml):
         f"{ach} GB/s")
     if sim.coef_classed():
         # bytes the class-id layout must move per sweep: 3 own-field reads and
-        # writes, 3 dual-field reads, 3 16-bit class ids per cell
-        ib = (9.0 * s + 6.0) * cells
+        # writes, 3 dual-field reads, 3 16-bit class ids per cell; in the
+        # one-launch half-steps also psi read and write and c_psi read of two
+        # components per slab cell (six slabs)
+        ib = (9.0 * s + 6.0) * cells + (6.0 * s * 6 * pml * n * n if int(fused) == 4 else 0.0)
         for k in ("update_h", "update_e"):
             if k in kernels:
                 kernels[k]["layout_bytes"] = ib
@@ -182,7 +188,7 @@ def run_device(sim, precision, warmup, steps, n, pml):
     res["cpml"] = {0: "separate slab launches", 1: "x/y slabs inside the Yee sweeps",
                    2: "z slabs inside the Yee sweeps, x/y slabs separate",
                    3: "every slab inside the single-pass step",
-                   4: "every slab inside the two Yee sweeps"}[int(fused)]
+                   4: "every slab inside the one-launch half-steps"}[int(fused)]
     sim.finish()
     return res
 

@@ -254,7 +254,8 @@ int xfd_read_td_nf2ff(xfd_ctx* ctx, int32_t n, int32_t d, int32_t which, double*
  * with the theta and the phi rows of the transform (transform.h:24-58).
  * k = 2 pi f / c.  e_node[a] (N_a + 1 values), h_node[a] and e_size[a] (N_a
  * values each) are the grid's node coordinates, cell centres and cell sizes
- * (GridSpace).  dst: na x 4 complex (A_theta, A_phi, F_theta, F_phi) as
+ * (GridSpace).  Several host threads may call it on one context: the calls
+ * wait for each other.  dst: na x 4 complex (A_theta, A_phi, F_theta, F_phi) as
  * interleaved (re, im) doubles. */
 int xfd_nf2ff_far_field(xfd_ctx* ctx, int32_t n, int32_t f, int32_t na, const double* theta, const double* phi,
                         const double* origin, double k, const double* const* e_node, const double* const* h_node,
@@ -322,11 +323,15 @@ int xfd_coef_layout(xfd_ctx* ctx, int32_t* classed, int64_t* classes);
  *     XFD_CPML_ZFUSED=1 keep the two sweeps.  XFD_STEP_CHUNK (1..1024)
  *     sets the i-planes each work-item marches.
  *   *fused = 4 (the default): each half-step is one launch that applies the
- *     update, every slab in boundary order per point (FP64 bitwise), the TFSF
- *     and lumped corrections and the point probes.  For 3D grids, dispersive
- *     ones included, whose slabs keep one order between every two axes, at
- *     most two per axis, and whose corrections lie off the far planes and
- *     outside the slabs (the reference applies those first).
+ *     update, every slab in boundary order per point (FP64 bitwise; FP32 rows
+ *     on which mode 2 would take the z slabs correct z first, as it does), the
+ *     TFSF and lumped corrections and the point probes.  For 3D grids, and 2D
+ *     ones whose Ex, Ey and Hz stay zero, whose slabs keep one order between
+ *     every two axes, at most two per axis, and whose corrections lie off the
+ *     far planes and outside the slabs (the reference applies those first).
+ *     Large dispersive grids, where it is slower, take it for the H half-step
+ *     alone (still reported as 4) or not at all; XFD_ADE_E=half / apart
+ *     selects.
  *     XFD_CPML_INSWEEP=0 or XFD_STEP_FUSED=0 turn it off; XFD_CPML_FUSED=1 and
  *     XFD_CPML_ZFUSED=1 select their own mode instead.
  * Modes 1 and 2 never with ADE materials or when a TFSF or lumped correction

@@ -31,6 +31,8 @@
 // 203 x 181 x 225, FP64), as were registers capped for one more wavefront per
 // SIMD (spills: 384^3 690 a half-step).  Loading plane i + 1 during plane i was tried: no
 // faster on small boxes and 2 % slower at 384^3 (fewer wavefronts per CU).
+// HBM at 384^3: 3.15 GB a half-step (FP32) at 5.9 TB/s, 5.74 GB (FP64) at 5.7, 1.2
+// times the compulsory bytes.
 #pragma once
 
 #include <climits>

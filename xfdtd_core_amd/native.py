@@ -393,7 +393,8 @@ class Simulation:
         1 the leading x/y slabs (XFD_CPML_FUSED=1), 2 the z slabs
         (XFD_CPML_ZFUSED=1, or FP32 with nz > 128 where 4 does not apply), 3
         all in the single-pass step (XFD_STEP_FUSED=1), 4 all, with the other
-        corrections, in one launch per half-step (the default)."""
+        corrections, in one launch per half-step (the default; on large
+        dispersive grids H alone, or 0)."""
         return int(self._L.xfd_sim_cpml_fused(self._h))
 
     def coef_classed(self) -> bool:
